@@ -78,10 +78,9 @@ def _log_int(rng, lo, hi):
 
 
 def _size(rng, lo, hi):
-    """A grid side lo..hi the multigrid can halve down to an odd factor 3, 5
-    or 7 or a power of two."""
+    """A grid side lo..hi that halves down to 4 or 3 (the coarsest level)."""
     while True:
-        s = rng.choice((1, 1, 1, 3, 5, 7)) << rng.randrange(3, 12)
+        s = rng.choice((1, 1, 3)) << rng.randrange(3, 12)
         if lo <= s <= hi:
             return s
 
@@ -96,7 +95,7 @@ def draw(rng):
         c["order"] = rng.choice((5, 5, 5, 3, 4))
         c["steps"] = rng.choice((2, 4, 8))
         ny = _size(rng, 64, 512)
-        c.update(nx=ny * rng.choice((1, 1, 2)), ny=ny)
+        c.update(nx=ny * rng.choice((2, 2, 3, 4)) // 2, ny=ny)
         if geometry == "disc" or big and geometry == "perio":
             c["geometry"] = "closed" if big else geometry
         if kind == "steps":
@@ -105,7 +104,7 @@ def draw(rng):
         return c
     if kind in ("solve", "twov"):
         ny = _size(rng, 64, 512)
-        c.update(nx=ny * rng.choice((1, 1, 2)), ny=ny)
+        c.update(nx=ny * rng.choice((2, 2, 3, 4)) // 2, ny=ny)
         return c
     if kind == "rhs":
         c["order"] = rng.choice((5, 5, 3, 1, 2, 4, 6))
