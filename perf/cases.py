@@ -85,6 +85,11 @@ def _size(rng, lo, hi):
             return s
 
 
+def _width(rng, ny):
+    # 3:2 halves down with powers of two only
+    return ny * rng.choice((2, 2, 4, 4 if ny % 3 == 0 else 3)) // 2
+
+
 def draw(rng):
     kind = rng.choice(("steps", "steps", "steps", "loop", "solve", "twov", "rhs", "mg", "diag"))
     geometry = rng.choice(("perio", "closed", "xchannel", "disc"))
@@ -95,7 +100,7 @@ def draw(rng):
         c["order"] = rng.choice((5, 5, 5, 3, 4))
         c["steps"] = rng.choice((2, 4, 8))
         ny = _size(rng, 64, 512)
-        c.update(nx=ny * rng.choice((2, 2, 3, 4)) // 2, ny=ny)
+        c.update(nx=_width(rng, ny), ny=ny)
         if geometry == "disc" or big and geometry == "perio":
             c["geometry"] = "closed" if big else geometry
         if kind == "steps":
@@ -104,7 +109,7 @@ def draw(rng):
         return c
     if kind in ("solve", "twov"):
         ny = _size(rng, 64, 512)
-        c.update(nx=ny * rng.choice((2, 2, 3, 4)) // 2, ny=ny)
+        c.update(nx=_width(rng, ny), ny=ny)
         return c
     if kind == "rhs":
         c["order"] = rng.choice((5, 5, 3, 1, 2, 4, 6))
