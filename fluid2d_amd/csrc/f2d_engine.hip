@@ -13,8 +13,10 @@
 //                prolongation and correction) or I(xc) (hierarchy.py:145-151)
 //   k_resid_restrict  residual + fill + full weighting + coarse fill
 //                (hierarchy.py:105-108), optional residual store and norms
-//   k_coarse     all levels below the fine part of one instance in one
-//                workgroup, operands in LDS (V-cycle or F-cycle tail)
+//   k_coarse_reg all levels below the fine part of one instance in one
+//                workgroup, operators in registers (V-cycle or F-cycle tail)
+//   k_coarse     the same for hierarchies outside its level slots, operands
+//                in LDS
 //   k_ortho      computeorthogradient (core/fortran_operators.f90:2-39)
 //   k_combine    final RK combination (core/timescheme.py:180)
 //   k_update, k_fold, k_npsum, k_finalize_psi, k_diag: solve control,
@@ -31,6 +33,7 @@
 #include <vector>
 
 #include "../../include/fluid2d_amd.h"
+#include "f2d_coarse.h"
 #include "f2d_dev.h"
 #include "f2d_engine.h"
 
@@ -2380,6 +2383,44 @@ __global__ void __launch_bounds__(COARSE_THREADS) k_coarse(const Task* __restric
 #endif
 }
 
+// The same levels with their operator rows in registers (f2d_coarse.h), for
+// the hierarchies whose levels fit its slots.
+template <typename T, bool S0, int MODE>
+__global__ void __launch_bounds__(256) k_coarse_reg(const Task* __restrict__ tasks,
+                                                    const coarse::Desc* __restrict__ dc,
+                                                    const double* __restrict__ pk, T* Q,
+                                                    const DynD* __restrict__ dyn, int pred,
+                                                    int inst_first, int first) {
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  const int ti = task_index();
+  const int inst = inst_first >= 0 ? inst_first + ti : tasks[ti].inst;
+#ifdef F2D_PHASE_STAMPS
+  Sync sy;
+  sy.tid = threadIdx.x;
+  sy.ck = 0;
+  if (threadIdx.x == 0 && blockIdx.x == 0) {
+    coarse_stamps[MODE][254] = wall_clock64();
+    coarse_stamps[MODE][255] = 100 + dc[inst].deep - dc[inst].top + 1;
+  }
+  F2D_CSTAMP(sy, MODE, 0);
+  auto stamp = [&](int code) {
+    F2D_CSTAMP(sy, MODE, code);
+    if (code == 2 && threadIdx.x == 0 && blockIdx.x == 0) {
+      coarse_stamps[MODE][252] = wall_clock64();
+      coarse_stamps[MODE][253] = 102;
+    }
+  };
+#else
+  auto stamp = [](int) {};
+#endif
+  // read here, not where the result is stored: a memory round trip there
+  long long xo = tasks[ti].xout;
+  asm volatile("" : "+s"(xo));
+  coarse::coarse_body<T, S0, MODE>(dc[inst], pk + (size_t)inst * coarse::PACK_VALUES, first,
+                                   Q + xo, (LDSP double*)lds_raw,
+                                   [&]() { return skip(dyn, inst, pred); }, stamp);
+}
+
 // ---------------------------------------------------------------------------
 // k_ortho: (u,v) from psi on [1, m-2] (computeorthogradient)
 // ---------------------------------------------------------------------------
@@ -2969,6 +3010,7 @@ struct Launch {
   int bar = 0;               // persistent launch: barrier slot
   int slot_off = 0;          // npsum slots
   size_t shmem = 0;          // k_coarse dynamic LDS
+  int creg = 0;              // coarse: 0 generic kernel, else 1 + the first slot of the register kernel
   int ty = TY;               // fine tile rows of k_smooth (k_resid_restrict: ty / 2 coarse rows)
   int maxite = -1;           // k_fold stopping test (< 0: the batch's full-solve values)
   double tol = 0.;
@@ -2982,6 +3024,10 @@ struct HostInst {
   long long buf[MAXLEV][2];  // x buffers per level (level 0 set per phase)
   size_t coarse_lds = 0;
   std::vector<int8_t> hmsk;  // cell mask (host copy): tile classification
+  bool creg = false;         // the coarse levels fit the register kernel's slots
+  coarse::Desc cd;           // its descriptor
+  std::vector<double> cA[MAXLEV];  // operator and mask of the levels it may take
+  std::vector<int8_t> cM[MAXLEV];
 };
 
 struct Batch {
@@ -2993,6 +3039,8 @@ struct Batch {
   int8_t* B = nullptr;
   size_t nP = 0, nQ = 0, nB = 0;
   InstD* dI = nullptr;
+  coarse::Desc* dC = nullptr;  // per instance: the register coarse kernel's levels
+  double* dPk = nullptr;       // and its packed operands, PACK_VALUES each
   DynD* dD = nullptr;
   DynD* hD = nullptr;  // pinned mirror
   Task* dT = nullptr;
@@ -3059,6 +3107,12 @@ constexpr double RR_SMALL_TILES = 64.;
 // two-level restrictions of b: launches of at most RB2_TILES tiles of 8
 // output rows take tiles of RB2_TY_SMALL rows
 constexpr int RB2_TILES = 256, RB2_TY_SMALL = 4;
+
+// the register coarse kernel: levels of at most COARSE_CELLS cells (halo
+// included) keep host copies of operator and mask, from which its operands
+// are packed
+constexpr int COARSE_TOP_CELLS = 2048;  // most cells of its top level
+constexpr size_t COARSE_CELLS = (size_t)(64 + 2 * NH) * (64 + 2 * NH);
 
 // ---- task helpers ----------------------------------------------------------
 static Task mk_task(int inst, int lev, int y0, int x0) {
@@ -3401,10 +3455,17 @@ struct Builder {
 
   void coarse(const std::vector<int>& who, int mode, int pred) {
     std::vector<Task> ts;
-    size_t sh = 0;
+    size_t sh = 0, shr = 0;
+    bool reg = true;
+    int first = coarse::NSLOT;
     for (int i : who) {
       HostInst& h = b.H[i];
       const int k = h.d.nfine;
+      reg = reg && h.creg;
+      if (h.creg) {
+        shr = std::max(shr, coarse::lds_values(h.cd) * sizeof(double));
+        first = std::min(first, h.cd.top);
+      }
       Task t = mk_task(i, k, 0, 0);
       h.cur[k] ^= 1;
       t.xout = h.buf[k][h.cur[k]];
@@ -3414,7 +3475,8 @@ struct Builder {
     Launch& L = add(L_COARSE, ts);
     L.mode = mode;
     L.pred = pred;
-    L.shmem = sh;
+    L.shmem = reg ? shr : sh;
+    L.creg = reg ? first + 1 : 0;
     // consecutive instances: the kernel takes instance first + task index
     L.inst0 = who.empty() ? -1 : who[0];
     for (size_t k = 0; k < who.size(); k++)
@@ -4020,6 +4082,22 @@ static int run_prog_t(Batch& b, const std::vector<Launch>& prog, ProfSel* prof =
                           b.partial);
         break;
       case L_COARSE:
+        if (L.creg > 0) {
+          // creg - 1: the first slot of the launch's instances
+          if (L.creg == 1 && L.mode == 0)
+            F2D_LAUNCH((k_coarse_reg<T, true, 0>), dim3(g), B1, L.shmem, b.s, TK, b.dC, b.dPk, Q,
+                       b.dD, L.pred, L.inst0, 0);
+          else if (L.creg == 1)
+            F2D_LAUNCH((k_coarse_reg<T, true, 1>), dim3(g), B1, L.shmem, b.s, TK, b.dC, b.dPk, Q,
+                       b.dD, L.pred, L.inst0, 0);
+          else if (L.mode == 0)
+            F2D_LAUNCH((k_coarse_reg<T, false, 0>), dim3(g), B1, L.shmem, b.s, TK, b.dC, b.dPk, Q,
+                       b.dD, L.pred, L.inst0, L.creg - 1);
+          else
+            F2D_LAUNCH((k_coarse_reg<T, false, 1>), dim3(g), B1, L.shmem, b.s, TK, b.dC, b.dPk, Q,
+                       b.dD, L.pred, L.inst0, L.creg - 1);
+          break;
+        }
         F2D_LAUNCH(k_coarse<T>, dim3(g), dim3(COARSE_THREADS), L.shmem, b.s, TK, b.dI, Q, b.B,
                            b.dD, L.pred, L.mode, b.coarse_wave_cells, L.inst0);
         break;
@@ -4286,6 +4364,8 @@ static void batch_free(Batch* b) {
   if (b->Q) (void)hipFree(b->Q);
   if (b->B) (void)hipFree(b->B);
   if (b->dI) (void)hipFree(b->dI);
+  if (b->dC) (void)hipFree(b->dC);
+  if (b->dPk) (void)hipFree(b->dPk);
   if (b->dD) (void)hipFree(b->dD);
   if (b->hD) (void)hipHostFree(b->hD);
   if (b->dT) (void)hipFree(b->dT);
@@ -4553,6 +4633,43 @@ static int extent_check(const f2d_model_params& p, size_t tsz) {
   return F2D_OK;
 }
 
+// The register coarse kernel's descriptor of levels k0 .. nlev - 1 of an
+// instance and its packed operands (pk, zero on entry); creg false where they
+// do not fit its slots.
+static void coarse_desc(const Batch& b, HostInst& h, int k0, double* pk) {
+  const InstD& d = h.d;
+  memset(&h.cd, 0, sizeof h.cd);
+  int M[MAXLEV], N[MAXLEV];
+  for (int l = 0; l < d.nlev; l++) {
+    M[l] = d.L[l].m - 2 * NH;
+    N[l] = d.L[l].n - 2 * NH;
+  }
+  coarse::Desc& c = h.cd;
+  h.creg = coarse::slots(k0, d.nlev, M, N, COARSE_TOP_CELLS, &c.top, &c.deep);
+  if (!h.creg) return;
+  const size_t tsz = b.prec == 0 ? sizeof(double) : sizeof(float);
+  int v = 0;
+  for (int l = k0, s = c.top; l < d.nlev; l++, s++) {
+    coarse::Slot& q = c.s[s];
+    q.M = M[l];
+    q.N = N[l];
+    q.lds = v;
+    v += 2 * M[l] * (s >= 3 ? coarse::PW : coarse::PB);
+    const double* A = h.cA[l].data();
+    const int8_t* mf = h.cM[l].data();
+    const int8_t* mc = l + 1 < d.nlev ? h.cM[l + 1].data() : nullptr;
+    switch (s) {
+      case 0: coarse::pack_slot<0>(pk, A, mf, M[l], N[l], mc, d.omega); break;
+      case 1: coarse::pack_slot<1>(pk, A, mf, M[l], N[l], mc, d.omega); break;
+      case 2: coarse::pack_slot<2>(pk, A, mf, M[l], N[l], mc, d.omega); break;
+      case 3: coarse::pack_slot<3>(pk, A, mf, M[l], N[l], mc, d.omega); break;
+      default: coarse::pack_slot<4>(pk, A, mf, M[l], N[l], mc, d.omega); break;
+    }
+  }
+  c.b = (const char*)b.Q + (size_t)d.L[k0].b * tsz;
+  c.omega = d.omega;
+}
+
 // apply a tuning: coarse split per instance, tile policy, programs rebuilt
 static int apply_tuning(Batch& b, const f2d_batch_tuning* t) {
   const size_t budget = lds_budget(t ? t->coarse_lds_budget : 0);
@@ -4560,10 +4677,20 @@ static int apply_tuning(Batch& b, const f2d_batch_tuning* t) {
   const size_t tsz = b.prec == 0 ? sizeof(double) : sizeof(float);
   for (int i = 0; i < b.ninst; i++) ETRY(first_coarse_level(b.H[i].d, budget, tsz, &k0[i]));
   size_t maxlds = 0;
+  bool all = true;  // every launch runs the register kernel
+  std::vector<coarse::Desc> cd(b.ninst);
+  std::vector<double> pk((size_t)b.ninst * coarse::PACK_VALUES, 0.);
+  for (int i = 0; i < b.ninst; i++) {
+    coarse_desc(b, b.H[i], k0[i], &pk[(size_t)i * coarse::PACK_VALUES]);
+    cd[i] = b.H[i].cd;
+    all = all && b.H[i].creg;
+  }
+  if (!b.dC) ECHK(hipMalloc(&b.dC, b.ninst * sizeof(coarse::Desc)));
+  if (!b.dPk) ECHK(hipMalloc(&b.dPk, pk.size() * sizeof(double)));
   for (int i = 0; i < b.ninst; i++) {
     b.H[i].d.nfine = k0[i];
     b.H[i].coarse_lds = coarse_bytes(b.H[i].d, k0[i], tsz);
-    maxlds = std::max(maxlds, b.H[i].coarse_lds);
+    if (!all) maxlds = std::max(maxlds, b.H[i].coarse_lds);
   }
   b.min_tiles = t ? std::max(0, t->min_tiles) : 0;
   b.persist = t ? std::max(0, t->persist) : 0;
@@ -4573,10 +4700,26 @@ static int apply_tuning(Batch& b, const f2d_batch_tuning* t) {
     const void* fn = b.prec == 0 ? (const void*)k_coarse<double> : (const void*)k_coarse<float>;
     ECHK(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)maxlds));
   }
+  size_t reglds = 0;
+  for (int i = 0; i < b.ninst; i++)
+    if (b.H[i].creg)
+      reglds = std::max(reglds, coarse::lds_values(b.H[i].cd) * sizeof(double));
+  if (reglds > 65536) {
+    const void* fn[8] = {
+        (const void*)k_coarse_reg<double, false, 0>, (const void*)k_coarse_reg<double, true, 0>,
+        (const void*)k_coarse_reg<double, false, 1>, (const void*)k_coarse_reg<double, true, 1>,
+        (const void*)k_coarse_reg<float, false, 0>,  (const void*)k_coarse_reg<float, true, 0>,
+        (const void*)k_coarse_reg<float, false, 1>,  (const void*)k_coarse_reg<float, true, 1>};
+    for (int q = 0; q < 4; q++)
+      ECHK(hipFuncSetAttribute(fn[4 * b.prec + q], hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)reglds));
+  }
   std::vector<InstD> di(b.ninst);
   for (int i = 0; i < b.ninst; i++) di[i] = b.H[i].d;
   drop_graph(b);
   ECHK(hipMemcpy(b.dI, di.data(), b.ninst * sizeof(InstD), hipMemcpyHostToDevice));
+  ECHK(hipMemcpy(b.dC, cd.data(), b.ninst * sizeof(coarse::Desc), hipMemcpyHostToDevice));
+  ECHK(hipMemcpy(b.dPk, pk.data(), pk.size() * sizeof(double), hipMemcpyHostToDevice));
   return build_programs(b);
 }
 
@@ -4814,6 +4957,17 @@ int f2d_batch_create(int ninst, const f2d_model_params* params, const int8_t* co
           ok = ok && hipMemcpy(b->B + d.sb0, bits.data(), S, hipMemcpyHostToDevice) == hipSuccess;
       }
       if (l > 0) ok = ok && hipMemcpy(b->B + d.L[l].msk, gm, S, hipMemcpyDeviceToDevice) == hipSuccess;
+      if (l > 0 && S <= COARSE_CELLS) {  // host copies for the packed coarse operands
+        std::vector<double>& cA = h.cA[l];
+        std::vector<int8_t>& cM = h.cM[l];
+        cA.resize(5 * S);
+        cM.resize(S);
+        ok = ok &&
+             hipMemcpy(cA.data(), gA, 5 * S * sizeof(double), hipMemcpyDeviceToHost) == hipSuccess &&
+             hipMemcpy(cM.data(), gm, S, hipMemcpyDeviceToHost) == hipSuccess;
+        if (b->prec != 0)  // the pool's rounding
+          for (double& a : cA) a = (double)(float)a;
+      }
       if (!ok) {
         f2d_gmg_free_raw(g);
         return bail(efail(F2D_E_HIP, "level copy"));
