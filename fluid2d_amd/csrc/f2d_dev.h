@@ -338,6 +338,138 @@ __device__ __forceinline__ double noslip_source_at(const int8_t* msk, const doub
   return r;
 }
 
+// NumPy's pairwise sum of at most 128 values (numpy/_core/src/umath
+// loops_utils.h.src): eight accumulators, or one below 8 values; element q
+// of the flattened interior of width N, arrays of row length n.  With N a
+// multiple of 8 a group of eight lies in one row (every start here is a
+// multiple of 8).
+__device__ __forceinline__ double np_leaf(const double* x, int n, int N, uint32_t s, uint32_t cnt) {
+  const uint32_t row = s / (uint32_t)N;
+  int col = (int)(s - row * (uint32_t)N);
+  const double* p = x + (size_t)(row + NH) * n + NH + col;
+  const bool aligned = (N & 7) == 0;
+  auto next = [&]() {
+    const double v = *p++;
+    if (++col == N) {
+      col = 0;
+      p += 2 * NH;
+    }
+    return v;
+  };
+  auto group = [&](double* v) {
+    if (aligned) {
+#pragma unroll
+      for (int q = 0; q < 8; q++) v[q] = p[q];
+      p += 8;
+      col += 8;
+      if (col == N) {
+        col = 0;
+        p += 2 * NH;
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < 8; q++) v[q] = next();
+    }
+  };
+  if (cnt < 8) {
+    double r = -0.0;
+    for (uint32_t k = 0; k < cnt; k++) r += next();
+    return r;
+  }
+  double a[8];
+  group(a);
+  uint32_t k = 8;
+  for (; k + 32 <= cnt; k += 32) {  // four groups in flight
+    double v[4][8];
+#pragma unroll
+    for (int g = 0; g < 4; g++) group(v[g]);
+#pragma unroll
+    for (int g = 0; g < 4; g++)
+#pragma unroll
+      for (int q = 0; q < 8; q++) a[q] += v[g][q];
+  }
+  for (; k + 8 <= cnt; k += 8) {
+    double v[8];
+    group(v);
+#pragma unroll
+    for (int q = 0; q < 8; q++) a[q] += v[q];
+  }
+  double r = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+  for (; k < cnt; k++) r += next();
+  return r;
+}
+
+// NumPy's pairwise sum of one chunk of at most 8192 values (NumPy's buffer)
+// by one wavefront; the result is lane 0's.  Six halvings (h = c / 2 less
+// c / 2 mod 8, while c > 128) give each lane one node of the recursion, which
+// is a leaf or two leaves; the nodes are then added up the same tree.
+// What bounds it: the memory round trips of one leaf, four groups of eight
+// at a time: 2048 x 1024 values 9.7 us (one thread per chunk with the
+// recursion on a stack took 1000); a chunk the halvings do not divide evenly
+// costs the same.
+__device__ __forceinline__ double np_chunk_wave(const double* x, int n, int N, uint32_t s0,
+                                                uint32_t cnt, int lane) {
+  uint32_t s = s0, c = cnt;
+  unsigned split = 0;  // bit d: the node at depth d on this lane's path splits
+  bool mine = true;    // the lane stands for a node (its remaining path bits are 0)
+#pragma unroll
+  for (int d = 0; d < 6; d++) {
+    const int bit = (lane >> (5 - d)) & 1;
+    if (c > 128) {
+      split |= 1u << d;
+      uint32_t h = c / 2;
+      h -= h % 8;
+      s += bit ? h : 0;
+      c = bit ? c - h : h;
+    } else if (bit) {
+      mine = false;
+    }
+  }
+  double r = 0.;
+  if (mine) {
+    if (c <= 128) {
+      r = np_leaf(x, n, N, s, c);
+    } else {
+      uint32_t h = c / 2;
+      h -= h % 8;
+      r = np_leaf(x, n, N, s, h);
+      r = r + np_leaf(x, n, N, s + h, c - h);
+    }
+  }
+#pragma unroll
+  for (int d = 5; d >= 0; d--) {
+    const double o = __shfl_down(r, 1u << (5 - d), 64);
+    if (((split >> d) & 1) && (lane & ((1 << (6 - d)) - 1)) == 0) r = r + o;
+  }
+  return r;
+}
+
+// 0 + v[0] + v[1] + ... in order, v global, by a 256-thread workgroup: tiles
+// of 256 through LDS, thread 0 adds (its loads no longer wait on memory one
+// by one).  The result is thread 0's.
+__device__ __forceinline__ double serial_sum256(const double* v, int cnt, int tid) {
+  __shared__ double sh[256];
+  double acc = 0.;
+  for (int b = 0; b < cnt; b += 256) {
+    if (b + tid < cnt) sh[tid] = v[b + tid];
+    __syncthreads();
+    if (tid == 0) {
+      const int e = cnt - b < 256 ? cnt - b : 256;
+      int k = 0;
+      for (; k + 16 <= e; k += 16) {
+        double t[16];
+#pragma unroll
+        for (int q = 0; q < 16; q++) t[q] = sh[k + q];
+#pragma unroll
+        for (int q = 0; q < 16; q++) acc = acc + t[q];
+      }
+      for (; k < e; k++) acc = acc + sh[k];
+    }
+    __syncthreads();
+  }
+  return acc;
+}
+
 // Calls f(j, i) at interior (J, I) and at each of its periodic halo images
 // (the positions store_img_mask32 writes).
 template <typename F>

@@ -2665,69 +2665,8 @@ __global__ void __launch_bounds__(256) k_flat_ops(const Task* __restrict__ tasks
 // ---------------------------------------------------------------------------
 // reductions
 // ---------------------------------------------------------------------------
-// NumPy pairwise sum of interior elements [s, s+cnt) (flattened C order)
-template <typename T>
-__device__ double np_pairwise_flat(const T* x, int n, int N, size_t start, size_t cnt) {
-  struct Fr {
-    size_t s, c;
-    double left;
-    int stage;
-  };
-  Fr st[16];
-  int sp = 0;
-  st[0] = {start, cnt, 0., 0};
-  double ret = 0.;
-  auto val = [&](size_t q) { return (double)x[at(NH + (int)(q / N), NH + (int)(q % N), n)]; };
-  while (sp >= 0) {
-    Fr& f = st[sp];
-    if (f.c <= 128) {
-      double r;
-      if (f.c < 8) {
-        r = -0.0;
-        for (size_t k = 0; k < f.c; k++) r += val(f.s + k);
-      } else {
-        double a[8];
-        for (int k = 0; k < 8; k++) a[k] = val(f.s + k);
-        size_t k;
-        for (k = 8; k < f.c - (f.c % 8); k += 8)
-          for (int q = 0; q < 8; q++) a[q] += val(f.s + k + q);
-        r = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
-        for (; k < f.c; k++) r += val(f.s + k);
-      }
-      ret = r;
-      sp--;
-      while (sp >= 0) {
-        Fr& pp = st[sp];
-        if (pp.stage == 1) {
-          pp.left = ret;
-          pp.stage = 2;
-          size_t h = pp.c / 2;
-          h -= h % 8;
-          st[++sp] = {pp.s + h, pp.c - h, 0., 0};
-          break;
-        } else {
-          ret = pp.left + ret;
-          sp--;
-        }
-      }
-      continue;
-    }
-    size_t h = f.c / 2;
-    h -= h % 8;
-    f.stage = 1;
-    st[sp + 1] = {f.s, h, 0., 0};
-    sp++;
-  }
-  return ret;
-}
-
-// One wavefront per 8192-element chunk of psi's interior (task.y0 = first
-// chunk, task.x0 = chunk count, one block per task with 64 threads per
-// chunk).  When the chunk length is 128 * 2^k -- every chunk of a
-// power-of-two grid -- NumPy's recursion splits it into equal halves down to
-// 128-element leaves, so lane L sums leaf L with NumPy's eight-accumulator
-// loop and the leaves are combined as the same balanced tree.  Other
-// lengths run NumPy's recursion on lane 0.
+// One wavefront per 8192-element chunk of psi's interior (np_chunk_wave;
+// task.y0 = first chunk, task.x0 = chunk count, at most four per block)
 __global__ void __launch_bounds__(256) k_npsum(const Task* __restrict__ tasks,
                                                const InstD* __restrict__ I, double* P,
                                                double* partial, const int* __restrict__ slot,
@@ -2742,32 +2681,11 @@ __global__ void __launch_bounds__(256) k_npsum(const Task* __restrict__ tasks,
   if (!src && !in.perio) return;
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int m = in.m, n = in.n, N = n - 2 * NH;
-  const size_t tot = (size_t)(m - 2 * NH) * N;
+  const uint32_t tot = (uint32_t)(m - 2 * NH) * (uint32_t)N;
   const double* psi = src ? in.nsrc : P + in.state + (size_t)m * n;
   for (int ch = wv; ch < tk.x0; ch += blockDim.x >> 6) {
-    const size_t s0 = (size_t)(tk.y0 + ch) * 8192;
-    const size_t cnt = tot - s0 < 8192 ? tot - s0 : 8192;
-    const size_t leaves = cnt / 128;
-    const bool balanced = cnt >= 128 && cnt % 128 == 0 && (leaves & (leaves - 1)) == 0;
-    double r = 0.;
-    if (!balanced) {
-      if (lane == 0) r = np_pairwise_flat<double>(psi, n, N, s0, cnt);
-    } else {
-      if ((size_t)lane < leaves) {
-        const size_t b0 = s0 + (size_t)lane * 128;
-        auto val = [&](size_t q) { return psi[at(NH + (int)(q / N), NH + (int)(q % N), n)]; };
-        double a[8];
-        for (int k = 0; k < 8; k++) a[k] = val(b0 + k);
-        for (int k = 8; k < 128; k += 8)
-          for (int q = 0; q < 8; q++) a[q] += val(b0 + k + q);
-        r = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
-      }
-      // balanced tree: at width w, lane L (L % 2w == 0) adds lane L + w
-      for (size_t w = 1; w < leaves; w <<= 1) {
-        const double o = __shfl_down(r, (unsigned)w, 64);
-        if ((lane % (2 * w)) == 0) r = r + o;
-      }
-    }
+    const uint32_t s0 = (uint32_t)(tk.y0 + ch) * 8192u;
+    const double r = np_chunk_wave(psi, n, N, s0, min(tot - s0, 8192u), lane);
     if (lane == 0) partial[slot[tk.slot] + ch] = r;
   }
 }
@@ -2860,9 +2778,9 @@ __global__ void __launch_bounds__(256) k_fold(const FoldSpan* __restrict__ spans
   const FoldSpan sp = spans[blockIdx.x];
   if (sp.count == 0 || !d.run) return;
   if (what == 3 || what == 4) {
-    if (tid != 0 || (what == 3 && !I[inst].perio)) return;
-    double acc = 0.;
-    for (int k = 0; k < sp.count; k++) acc = acc + partial[sp.first + k];
+    if (what == 3 && !I[inst].perio) return;
+    const double acc = serial_sum256(partial + sp.first, sp.count, tid);
+    if (tid != 0) return;
     // domain_integration(z) = np.sum(interior) * 1. (core/grid.py:132-140)
     if (what == 3)
       d.psim = acc * 1. / I[inst].area;

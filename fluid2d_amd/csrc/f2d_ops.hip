@@ -6,6 +6,8 @@
 // sweep in FP64).  These are the building blocks; the fused/LDS-tiled
 // variants live in f2d_fused.hip.  Each kernel cites the reference routine
 // whose arithmetic (operation order included) it reproduces.
+#include <algorithm>
+
 #include "f2d_ops.h"
 #include "f2d_dev.h"
 
@@ -571,24 +573,38 @@ __device__ __forceinline__ T wave_max(T v) {
   return v;
 }
 
-// per-workgroup sums of NV quantities over interior cells: partial[blk*NV+k]
-template <int NV>
-__device__ __forceinline__ void block_reduce_store(double (&v)[NV], const bool (&is_max)[NV],
-                                                   double* partial) {
+// Per-workgroup partials of NV quantities over the interior cells:
+// partial[workgroup * NV + k].  Workgroups of (64, 4); workgroup (bx, by)
+// takes columns 512 bx .. and rows 4 by .., striding over the grid's extent
+// -- no division per cell (a flat index split by N cost three times the
+// memory time).  Bound by the memory: computekemaxu of 2048 x 1024 cells 11
+// us, 3.2 TB/s of u, v and the mask; computenorm 5.6 us.  cell(c, v)
+// adds cell c's values to v (a maximum where bit k of MAXES is set).
+constexpr int RED_COLS = 512, RED_ROWS = 4;
+template <int NV, unsigned MAXES, typename F>
+__device__ __forceinline__ void reduce_cells(int m, int n, double* partial, F cell) {
   __shared__ double sh[NV][4];
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  double v[NV];
+#pragma unroll
+  for (int k = 0; k < NV; k++) v[k] = 0.;
+  const int N = n - 2 * NH, M = m - 2 * NH;
+  for (int j = blockIdx.y * RED_ROWS + threadIdx.y; j < M; j += gridDim.y * RED_ROWS)
+    for (int i0 = blockIdx.x * RED_COLS; i0 < N; i0 += gridDim.x * RED_COLS)
+#pragma unroll 4
+      for (int i = i0 + threadIdx.x; i < min(i0 + RED_COLS, N); i += 64)
+        cell(at(NH + j, NH + i, n), v);
+#pragma unroll
   for (int k = 0; k < NV; k++) {
-    double w = is_max[k] ? wave_max(v[k]) : wave_sum(v[k]);
-    if (lane == 0) sh[k][wid] = w;
+    const double w = (MAXES >> k) & 1 ? wave_max(v[k]) : wave_sum(v[k]);
+    if (threadIdx.x == 0) sh[k][threadIdx.y] = w;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int k = 0; k < NV; k++) {
-      double a = sh[k][0];
-      for (int w = 1; w < (int)(blockDim.x >> 6); w++)
-        a = is_max[k] ? fmax(a, sh[k][w]) : a + sh[k][w];
-      partial[(size_t)blockIdx.x * NV + k] = a;
-    }
+  if (threadIdx.y == 0 && threadIdx.x < NV) {
+    const int k = threadIdx.x;
+    double a = sh[k][0];
+#pragma unroll
+    for (int w = 1; w < 4; w++) a = (MAXES >> k) & 1 ? fmax(a, sh[k][w]) : a + sh[k][w];
+    partial[((size_t)blockIdx.y * gridDim.x + blockIdx.x) * NV + k] = a;
   }
 }
 
@@ -596,17 +612,10 @@ __device__ __forceinline__ void block_reduce_store(double (&v)[NV], const bool (
 __global__ void __launch_bounds__(256) k_norm2_partial(const int8_t* __restrict__ msk,
                                                        const double* __restrict__ x, int m,
                                                        int n, double* partial) {
-  const int N = n - 2 * NH;
-  const size_t tot = (size_t)(m - 2 * NH) * N;
-  double acc = 0.;
-  for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < tot;
-       q += (size_t)gridDim.x * blockDim.x) {
-    const size_t c = at(NH + (int)(q / N), NH + (int)(q % N), n);
-    if (msk[c] != 0) acc += x[c] * x[c];
-  }
-  double v[1] = {acc};
-  const bool mx[1] = {false};
-  block_reduce_store<1>(v, mx, partial);
+  reduce_cells<1, 0>(m, n, partial, [&](size_t c, double* v) {
+    const double q = x[c];
+    if (msk[c] != 0) v[0] += q * q;
+  });
 }
 
 // diagnostics: {maxu, ke, sum w, sum w^2, d4, d5, d6, d7}
@@ -617,13 +626,9 @@ __global__ void __launch_bounds__(256) k_diag_partial(const int8_t* __restrict__
                                                       const double* __restrict__ xr,
                                                       const double* __restrict__ yr, int m,
                                                       int n, double* partial) {
-  const int N = n - 2 * NH;
-  const size_t tot = (size_t)(m - 2 * NH) * N, P = (size_t)m * n;
+  const size_t P = (size_t)m * n;
   const double *w = s, *psi = s + P, *u = s + 2 * P, *v = s + 3 * P, *f4 = s + 4 * P;
-  double a[8] = {0., 0., 0., 0., 0., 0., 0., 0.};
-  for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < tot;
-       q += (size_t)gridDim.x * blockDim.x) {
-    const size_t c = at(NH + (int)(q / N), NH + (int)(q % N), n);
+  reduce_cells<8, 1>(m, n, partial, [&](size_t c, double* a) {
     const int mk = msk[c];
     if (mk == 1) {
       const double zu = u[c] * u[c] + u[c - 1] * u[c - 1];
@@ -648,9 +653,7 @@ __global__ void __launch_bounds__(256) k_diag_partial(const int8_t* __restrict__
         a[6] += f4[c] * f4[c];
       }
     }
-  }
-  const bool mx[8] = {true, false, false, false, false, false, false, false};
-  block_reduce_store<8>(a, mx, partial);
+  });
 }
 
 // kemaxu alone: {ke, maxu}
@@ -658,21 +661,15 @@ __global__ void __launch_bounds__(256) k_kemaxu_partial(const int8_t* __restrict
                                                         const double* __restrict__ u,
                                                         const double* __restrict__ v, int m,
                                                         int n, double* partial) {
-  const int N = n - 2 * NH;
-  const size_t tot = (size_t)(m - 2 * NH) * N;
-  double a[2] = {0., 0.};
-  for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < tot;
-       q += (size_t)gridDim.x * blockDim.x) {
-    const size_t c = at(NH + (int)(q / N), NH + (int)(q % N), n);
+  reduce_cells<2, 2>(m, n, partial, [&](size_t c, double* a) {
+    const double uc = u[c], uw = u[c - 1], vc = v[c], vs = v[c - n];
     if (msk[c] == 1) {
-      const double zu = u[c] * u[c] + u[c - 1] * u[c - 1];
-      const double zv = v[c] * v[c] + v[c - n] * v[c - n];
+      const double zu = uc * uc + uw * uw;
+      const double zv = vc * vc + vs * vs;
       a[0] += zu + zv;
-      a[1] = fmax(a[1], fabs(u[c] + u[c - 1]) + fabs(v[c] + v[c - n]));
+      a[1] = fmax(a[1], fabs(uc + uw) + fabs(vc + vs));
     }
-  }
-  const bool mx[2] = {false, true};
-  block_reduce_store<2>(a, mx, partial);
+  });
 }
 
 // {sum s*a, sum s*b} over the interior where msk != 0
@@ -682,19 +679,12 @@ __global__ void __launch_bounds__(256) k_dot2_partial(const int8_t* __restrict__
                                                       const double* __restrict__ a,
                                                       const double* __restrict__ b, int m, int n,
                                                       double* partial) {
-  const int N = n - 2 * NH;
-  const size_t tot = (size_t)(m - 2 * NH) * N;
-  double acc[2] = {0., 0.};
-  for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < tot;
-       q += (size_t)gridDim.x * blockDim.x) {
-    const size_t c = at(NH + (int)(q / N), NH + (int)(q % N), n);
+  reduce_cells<2, 0>(m, n, partial, [&](size_t c, double* v) {
     if (msk[c] != 0) {
-      acc[0] += s[c] * a[c];
-      acc[1] += s[c] * b[c];
+      v[0] += s[c] * a[c];
+      v[1] += s[c] * b[c];
     }
-  }
-  const bool mx[2] = {false, false};
-  block_reduce_store<2>(acc, mx, partial);
+  });
 }
 
 // The three masked sums of core/fortran_diag.f90 over the interior:
@@ -706,119 +696,68 @@ __global__ void __launch_bounds__(256) k_msum_partial(const int8_t* __restrict__
                                                       const double* __restrict__ x,
                                                       const double* __restrict__ y, int m, int n,
                                                       double* partial) {
-  const int N = n - 2 * NH;
-  const size_t tot = (size_t)(m - 2 * NH) * N;
   constexpr int NV = KIND == 2 ? 2 : 1;
-  double acc[NV];
-  for (int k = 0; k < NV; k++) acc[k] = 0.;
-  for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < tot;
-       q += (size_t)gridDim.x * blockDim.x) {
-    const size_t c = at(NH + (int)(q / N), NH + (int)(q % N), n);
+  reduce_cells<NV, 0>(m, n, partial, [&](size_t c, double* v) {
     const int8_t mk = msk[c];
+    const double q = x[c];
     if constexpr (KIND == 0) {
-      if (mk != 0) acc[0] += x[c] * y[c];
+      const double p = y[c];
+      if (mk != 0) v[0] += q * p;
     } else if constexpr (KIND == 1) {
-      if (mk != 0) acc[0] += x[c];
+      if (mk != 0) v[0] += q;
     } else {
       if (mk == 1) {
-        acc[0] += x[c];
-        acc[NV - 1] += x[c] * x[c];
+        v[0] += q;
+        v[NV - 1] += q * q;
       }
     }
+  });
+}
+
+// Folds nblk partial rows of nv values (1, 2 or 8) in a fixed order: thread t
+// takes entries t, t + 256, ... (all of quantity t mod nv), then a tree over
+// the threads; scale[k] multiplies result k (diagnostic constants 0.25 /
+// 0.5).  Bound by two memory round trips: 3.2 us for 1024 rows (one thread
+// per quantity adding them one after another took 94).
+__global__ void __launch_bounds__(256) k_fold(const double* __restrict__ partial, int nblk,
+                                              int nv, MaxMask mm, Scale8 sc,
+                                              double* __restrict__ out) {
+  __shared__ double sh[256];
+  const int t = threadIdx.x, tot = nblk * nv;
+  const bool ismax = (mm.bits >> (t % nv)) & 1;
+  double a = 0.;
+  if (t < tot) a = partial[t];
+#pragma unroll 4
+  for (int e = t + 256; e < tot; e += 256) {
+    const double y = partial[e];
+    a = ismax ? fmax(a, y) : a + y;
   }
-  bool mx[NV];
-  for (int k = 0; k < NV; k++) mx[k] = false;
-  block_reduce_store<NV>(acc, mx, partial);
-}
-
-// fold nblk partial rows of NV values in block order; scale[k] multiplies
-// result k (diagnostic constants 0.25 / 0.5).
-__global__ void k_fold(const double* __restrict__ partial, int nblk, int nv, MaxMask mm,
-                       Scale8 sc, double* __restrict__ out) {
-  if (threadIdx.x >= (unsigned)nv) return;
-  const int k = threadIdx.x;
-  const bool ismax = (mm.bits >> k) & 1;
-  double a = partial[k];
-  for (int b = 1; b < nblk; b++) a = ismax ? fmax(a, partial[(size_t)b * nv + k]) : a + partial[(size_t)b * nv + k];
-  out[k] = a * sc.v[k];
-}
-
-// NumPy's pairwise sum of a contiguous run (numpy _core/src/umath
-// loops_utils.h.src pairwise_sum), on gathered interior elements.
-__device__ double np_pairwise_dev(const double* x, int n, int N, size_t start, size_t cnt) {
-  // explicit stack of (start, cnt, partial-state)
-  struct Fr {
-    size_t s, c;
-    double left;
-    int stage;
-  };
-  Fr st[16];
-  int sp = 0;
-  st[0] = {start, cnt, 0., 0};
-  double ret = 0.;
-  auto val = [&](size_t q) { return x[at(NH + (int)(q / N), NH + (int)(q % N), n)]; };
-  while (sp >= 0) {
-    Fr& f = st[sp];
-    if (f.c <= 128) {
-      double r;
-      if (f.c < 8) {
-        r = -0.0;
-        for (size_t k = 0; k < f.c; k++) r += val(f.s + k);
-      } else {
-        double a[8];
-        for (int k = 0; k < 8; k++) a[k] = val(f.s + k);
-        size_t k;
-        for (k = 8; k < f.c - (f.c % 8); k += 8)
-          for (int q = 0; q < 8; q++) a[q] += val(f.s + k + q);
-        r = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
-        for (; k < f.c; k++) r += val(f.s + k);
-      }
-      ret = r;
-      sp--;
-      // deliver to parent
-      while (sp >= 0) {
-        Fr& p = st[sp];
-        if (p.stage == 1) {  // left done, start right
-          p.left = ret;
-          p.stage = 2;
-          size_t h = p.c / 2;
-          h -= h % 8;
-          st[++sp] = {p.s + h, p.c - h, 0., 0};
-          break;
-        } else {  // right done
-          ret = p.left + ret;
-          sp--;
-        }
-      }
-      continue;
-    }
-    // split
-    size_t h = f.c / 2;
-    h -= h % 8;
-    f.stage = 1;
-    st[sp + 1] = {f.s, h, 0., 0};
-    sp++;
+  sh[t] = a;
+  __syncthreads();
+  // entries past tot hold 0, neutral for the sums and for the maxima of
+  // magnitudes
+  for (int h = 128; h >= nv; h >>= 1) {
+    if (t < h) sh[t] = ismax ? fmax(sh[t], sh[t + h]) : sh[t] + sh[t + h];
+    __syncthreads();
   }
-  return ret;
+  if (t < nv) out[t] = sh[t] * sc.v[t];
 }
 
-// one thread per 8192-element chunk of the flattened interior
-__global__ void k_npsum_chunks(const double* __restrict__ x, int m, int n, double* partial) {
+// NumPy's sum of the interior: one wavefront per 8192-value chunk
+// (np_chunk_wave), then the chunks in order
+__global__ void __launch_bounds__(64) k_npsum_chunks(const double* __restrict__ x, int m, int n,
+                                                     double* partial) {
   const int N = n - 2 * NH;
-  const size_t tot = (size_t)(m - 2 * NH) * N;
-  const size_t ch = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const size_t s = ch * 8192;
-  if (s >= tot) return;
-  const size_t cnt = tot - s < 8192 ? tot - s : 8192;
-  partial[ch] = np_pairwise_dev(x, n, N, s, cnt);
+  const uint32_t tot = (uint32_t)(m - 2 * NH) * (uint32_t)N;
+  const uint32_t s = blockIdx.x * 8192u;
+  const double r = np_chunk_wave(x, n, N, s, min(tot - s, 8192u), threadIdx.x);
+  if (threadIdx.x == 0) partial[blockIdx.x] = r;
 }
 // acc = 0 + chunk0 + chunk1 + ...; out[0] = acc * 1. / div (if div != 0)
-__global__ void k_npsum_fold(const double* __restrict__ partial, int nch, double div,
-                             double* out) {
-  if (threadIdx.x != 0) return;
-  double acc = 0.;
-  for (int k = 0; k < nch; k++) acc = acc + partial[k];
-  out[0] = div != 0. ? acc * 1. / div : acc;
+__global__ void __launch_bounds__(256) k_npsum_fold(const double* __restrict__ partial, int nch,
+                                                    double div, double* out) {
+  const double acc = serial_sum256(partial, nch, threadIdx.x);
+  if (threadIdx.x == 0) out[0] = div != 0. ? acc * 1. / div : acc;
 }
 
 // ---------------------------------------------------------------------------
@@ -998,70 +937,74 @@ void launch_coarse_mask(const int8_t* msk1, int8_t* msk2, int m2, int n2, int n1
                      n1);
 }
 
-static int red_blocks(int m, int n) {
-  const size_t tot = (size_t)(m - 2 * NH) * (n - 2 * NH);
-  size_t b = (tot + 255) / 256;
-  if (b > (size_t)kRedMaxBlocks) b = kRedMaxBlocks;
-  if (b < 1) b = 1;
-  return (int)b;
+// grid of reduce_cells: at most kRedMaxBlocks workgroups
+static dim3 red_grid(int m, int n) {
+  const int bx = std::min((n - 2 * NH + RED_COLS - 1) / RED_COLS, kRedMaxBlocks);
+  const int by = std::min((m - 2 * NH + RED_ROWS - 1) / RED_ROWS, kRedMaxBlocks / bx);
+  return dim3((unsigned)bx, (unsigned)by);
 }
 
 void launch_norm2(const int8_t* msk, const double* x, int m, int n, double* partial, double* out,
                   hipStream_t s) {
-  const int nb = red_blocks(m, n);
-  hipLaunchKernelGGL(k_norm2_partial, dim3(nb), B1, 0, s, msk, x, m, n, partial);
+  const dim3 g = red_grid(m, n);
+  const int nb = (int)(g.x * g.y);
+  hipLaunchKernelGGL(k_norm2_partial, g, B2, 0, s, msk, x, m, n, partial);
   Scale8 sc;
   for (int k = 0; k < 8; k++) sc.v[k] = 1.;
-  hipLaunchKernelGGL(k_fold, dim3(1), dim3(64), 0, s, partial, nb, 1, MaxMask{0}, sc, out);
+  hipLaunchKernelGGL(k_fold, dim3(1), B1, 0, s, partial, nb, 1, MaxMask{0}, sc, out);
 }
 void launch_kemaxu(const int8_t* msk, const double* u, const double* v, int m, int n,
                    double* partial, double* out, hipStream_t s) {
-  const int nb = red_blocks(m, n);
-  hipLaunchKernelGGL(k_kemaxu_partial, dim3(nb), B1, 0, s, msk, u, v, m, n, partial);
+  const dim3 g = red_grid(m, n);
+  const int nb = (int)(g.x * g.y);
+  hipLaunchKernelGGL(k_kemaxu_partial, g, B2, 0, s, msk, u, v, m, n, partial);
   Scale8 sc;
   for (int k = 0; k < 8; k++) sc.v[k] = 1.;
   sc.v[0] = 0.25;
   sc.v[1] = 0.5;
-  hipLaunchKernelGGL(k_fold, dim3(1), dim3(64), 0, s, partial, nb, 2, MaxMask{2}, sc, out);
+  hipLaunchKernelGGL(k_fold, dim3(1), B1, 0, s, partial, nb, 2, MaxMask{2}, sc, out);
 }
 void launch_diag(const int8_t* msk, const double* state, int kind, const double* xr,
                  const double* yr, int m, int n, double* partial, double* out, hipStream_t s) {
-  const int nb = red_blocks(m, n);
-  hipLaunchKernelGGL(k_diag_partial, dim3(nb), B1, 0, s, msk, state, kind, xr, yr, m, n, partial);
+  const dim3 g = red_grid(m, n);
+  const int nb = (int)(g.x * g.y);
+  hipLaunchKernelGGL(k_diag_partial, g, B2, 0, s, msk, state, kind, xr, yr, m, n, partial);
   Scale8 sc;
   for (int k = 0; k < 8; k++) sc.v[k] = 1.;
   sc.v[0] = 0.5;
   sc.v[1] = 0.25;
-  hipLaunchKernelGGL(k_fold, dim3(1), dim3(64), 0, s, partial, nb, 8, MaxMask{1}, sc, out);
+  hipLaunchKernelGGL(k_fold, dim3(1), B1, 0, s, partial, nb, 8, MaxMask{1}, sc, out);
 }
 void launch_dot2(const int8_t* msk, const double* x, const double* a, const double* b, int m,
                  int n, double* partial, double* out, hipStream_t s) {
-  const int nb = red_blocks(m, n);
-  hipLaunchKernelGGL(k_dot2_partial, dim3(nb), B1, 0, s, msk, x, a, b, m, n, partial);
+  const dim3 g = red_grid(m, n);
+  const int nb = (int)(g.x * g.y);
+  hipLaunchKernelGGL(k_dot2_partial, g, B2, 0, s, msk, x, a, b, m, n, partial);
   Scale8 sc;
   for (int k = 0; k < 8; k++) sc.v[k] = 1.;
-  hipLaunchKernelGGL(k_fold, dim3(1), dim3(64), 0, s, partial, nb, 2, MaxMask{0}, sc, out);
+  hipLaunchKernelGGL(k_fold, dim3(1), B1, 0, s, partial, nb, 2, MaxMask{0}, sc, out);
 }
 void launch_msum(int kind, const int8_t* msk, const double* x, const double* y, int m, int n,
                  double* partial, double* out, hipStream_t s) {
-  const int nb = red_blocks(m, n);
+  const dim3 g = red_grid(m, n);
+  const int nb = (int)(g.x * g.y);
   if (kind == 0)
-    hipLaunchKernelGGL(k_msum_partial<0>, dim3(nb), B1, 0, s, msk, x, y, m, n, partial);
+    hipLaunchKernelGGL(k_msum_partial<0>, g, B2, 0, s, msk, x, y, m, n, partial);
   else if (kind == 1)
-    hipLaunchKernelGGL(k_msum_partial<1>, dim3(nb), B1, 0, s, msk, x, y, m, n, partial);
+    hipLaunchKernelGGL(k_msum_partial<1>, g, B2, 0, s, msk, x, y, m, n, partial);
   else
-    hipLaunchKernelGGL(k_msum_partial<2>, dim3(nb), B1, 0, s, msk, x, y, m, n, partial);
+    hipLaunchKernelGGL(k_msum_partial<2>, g, B2, 0, s, msk, x, y, m, n, partial);
   Scale8 sc;
   for (int k = 0; k < 8; k++) sc.v[k] = 1.;
-  hipLaunchKernelGGL(k_fold, dim3(1), dim3(64), 0, s, partial, nb, kind == 2 ? 2 : 1, MaxMask{0},
+  hipLaunchKernelGGL(k_fold, dim3(1), B1, 0, s, partial, nb, kind == 2 ? 2 : 1, MaxMask{0},
                      sc, out);
 }
 void launch_domain_sum(const double* x, int m, int n, double div, double* partial, double* out,
                        hipStream_t s) {
   const size_t tot = (size_t)(m - 2 * NH) * (n - 2 * NH);
   const int nch = (int)((tot + 8191) / 8192);
-  hipLaunchKernelGGL(k_npsum_chunks, dim3((nch + 63) / 64), dim3(64), 0, s, x, m, n, partial);
-  hipLaunchKernelGGL(k_npsum_fold, dim3(1), dim3(64), 0, s, partial, nch, div, out);
+  hipLaunchKernelGGL(k_npsum_chunks, dim3(nch), dim3(64), 0, s, x, m, n, partial);
+  hipLaunchKernelGGL(k_npsum_fold, dim3(1), B1, 0, s, partial, nch, div, out);
 }
 
 template void launch_adv_upwind<double>(const int8_t*, const double*, double*, const double*,
