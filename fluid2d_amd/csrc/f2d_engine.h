@@ -93,5 +93,23 @@ struct Task {
   int slot;  // the task's index in its launch's list as built (partial-sum slot)
 };
 
+// A stand-alone hierarchy on the engine's kernels (f2d_gmg): level arrays of
+// the caller, captured graphs of two V-cycles from level 0 on its x (which
+// 0) and of an F-cycle of its b into its x (which 1).  t is scratch; levels
+// below the first coarse one are not written.  bits, w0: the finest operator
+// as stencil bits and weights.  A hierarchy the kernels do not take gives
+// null.
+struct HierLevel {
+  int m, n;
+  int8_t* msk;
+  double *A, *x, *b, *t;
+};
+struct Hierarchy;
+int hierarchy_create(int nlev, const HierLevel* L, const uint8_t* bits, const double* w0,
+                     double omega, Hierarchy** out);
+int hierarchy_run(Hierarchy* h, int which, hipStream_t s);
+void hierarchy_destroy(Hierarchy* h);
+const char* hierarchy_error();
+
 }  // namespace eng
 }  // namespace f2d

@@ -2941,7 +2941,19 @@ struct HostInst {
   int cur[MAXLEV];
   long long buf[MAXLEV][2];  // x buffers per level (level 0 set per phase)
   size_t coarse_lds = 0;
-  std::vector<int8_t> hmsk;  // cell mask (host copy): tile classification
+  // solid cells above and left of (j, i), (m + 1) x (n + 1): the tile
+  // classification counts those of a rectangle without walking it
+  std::vector<int> solid;
+  void count_solid(const int8_t* msk, int m, int n) {
+    solid.assign((size_t)(m + 1) * (n + 1), 0);
+    for (int j = 0; j < m; j++) {
+      int row = 0;
+      for (int i = 0; i < n; i++) {
+        row += msk[(size_t)j * n + i] == 0;
+        solid[(size_t)(j + 1) * (n + 1) + i + 1] = solid[(size_t)j * (n + 1) + i + 1] + row;
+      }
+    }
+  }
   bool creg = false;         // the coarse levels fit the register kernel's slots
   coarse::Desc cd;           // its descriptor
   std::vector<double> cA[MAXLEV];  // operator and mask of the levels it may take
@@ -2950,6 +2962,7 @@ struct HostInst {
 
 struct Batch {
   int ninst = 0;
+  bool hierarchy = false;  // the levels of a Gmg (its arrays, not the batch's), no model
   int prec = 0;  // 0: FP64 throughout; 1: FP32 tendencies and V-cycles
   std::vector<HostInst> H;
   double* P = nullptr;  // FP64 pool
@@ -3154,10 +3167,10 @@ struct Builder {
     // is placed in coarse coordinates, ty coarse rows of TX2 columns)
     const int j0 = rr ? 2 * t.y0 - 4 : t.y0 - 3, j1 = rr ? 2 * (t.y0 + ty) + 2 : t.y0 + ty + 3;
     const int i0 = rr ? 2 * t.x0 - 4 : t.x0 - 3, i1 = rr ? 2 * (t.x0 + TX2) + 2 : t.x0 + TX + 3;
-    for (int j = std::max(0, j0); j < std::min(m, j1); j++)
-      for (int i = std::max(0, i0); i < std::min(n, i1); i++)
-        if (h.hmsk[(size_t)j * n + i] == 0) return true;
-    return false;
+    const int a = std::max(0, j0), e = std::min(m, j1), c = std::max(0, i0), f = std::min(n, i1);
+    if (a >= e || c >= f) return false;
+    auto Z = [&](int j, int i) { return h.solid[(size_t)j * (n + 1) + i]; };
+    return Z(e, f) - Z(a, f) - Z(e, c) + Z(a, c) > 0;
   }
   // Reorder each XCD's share of a launch's tasks (task_index gives XCD x a
   // contiguous share; its first workgroups land on distinct CUs) so that
@@ -3513,6 +3526,96 @@ struct Builder {
     ortho(who, [k](HostInst& h) { return h.d.k[k]; }, 2, [k](HostInst& h) { return h.d.kp[k]; });
   }
 
+  // F-cycle from level 0 (hierarchy.py:131-151) whose b1 is formed: b
+  // restricted down the fine levels.
+  // Level l = nfine - 1 - dd of an instance goes to l + 1 at
+  // bottom-aligned step dd; steps dd and dd - 1 share a k_restrict_b2
+  // launch (one-level launches where the program's mid-level phases
+  // are merged into persistent launches)
+  void fcycle_down(const std::vector<int>& who, int pred) {
+    int Dmax = 0;
+    for (int i : who) Dmax = std::max(Dmax, b.H[i].d.nfine - 1);
+    for (int dd = Dmax - 1; dd >= 0; dd -= (b.persist > 0 ? 1 : 2)) {
+      if (b.persist > 0) {
+        double cells = 0.;
+        for (int i : who) {
+          const int l = b.H[i].d.nfine - 1 - dd;
+          if (l >= 1) cells += (double)(b.H[i].d.L[l].m - 2 * NH) * (b.H[i].d.L[l].n - 2 * NH);
+        }
+        const int ty = pick_ty_cells(cells);
+        std::vector<Task> rs;
+        for (int i : who) {
+          const int l = b.H[i].d.nfine - 1 - dd;
+          if (l >= 1) rr_tasks(i, l, 0, -1, -1, rs, ty / 2);
+        }
+        if (!rs.empty()) {
+          Launch& L = add(L_RR, rs);
+          L.flags = 2;
+          L.pred = pred;
+          L.ty = ty;
+        }
+        continue;
+      }
+      // output tiles of 8 rows, or of RB2_TY_SMALL rows where 8 would give
+      // at most RB2_TILES tiles (latency-bound launches: more, shorter tiles)
+      std::vector<Task> rs;
+      int rty = 8;
+      for (int ty : {8, RB2_TY_SMALL}) {
+        rs.clear();
+        rty = ty;
+        for (int i : who) {
+          const int l = b.H[i].d.nfine - 1 - dd;
+          if (dd >= 1 && l >= 1)
+            rb_tasks(i, l, 2, rs, ty);
+          else if (dd >= 1 && l == 0)
+            rb_tasks(i, 1, 1, rs, ty);
+          else if (dd == 0 && l >= 1)
+            rb_tasks(i, l, 1, rs, ty);
+        }
+        if (ty == 8 && (int)rs.size() > RB2_TILES) break;
+      }
+      if (!rs.empty()) {
+        Launch& L = add(L_RB2, rs);
+        L.pred = pred;
+        L.ty = rty;
+      }
+    }
+  }
+  // the V-cycles of an F-cycle, from each fine level upward
+  void fcycle_up(const std::vector<int>& who, int pred) {
+    int Dmax = 0;
+    for (int i : who) Dmax = std::max(Dmax, b.H[i].d.nfine - 1);
+    for (int dd = 0; dd <= Dmax; dd++) {
+      std::vector<int> sub, st(b.ninst, 0);
+      for (int i : who)
+        if (b.H[i].d.nfine - 1 >= dd) {
+          sub.push_back(i);
+          st[i] = b.H[i].d.nfine - 1 - dd;
+        }
+      vcycle(sub, st, 3, pred, false);
+    }
+  }
+
+  // the two programs of a stand-alone hierarchy (Gmg): two V-cycles from
+  // level 0 on its x (hierarchy.py:207-218), and an F-cycle of its b
+  void hierarchy_programs() {
+    HostInst& h = b.H[0];
+    const std::vector<int> who{0}, st{0};
+    prog = &b.prog_step;
+    vcycle(who, st, 0, 0, false);
+    vcycle(who, st, 0, 0, false);
+    prog = &b.prog_init;
+    std::vector<Task> rs;
+    rr_tasks(0, 0, 0, -1, -1, rs, pick_ty_cells((double)h_cells(0)) / 2);
+    Launch& L = add(L_RR, rs);
+    L.flags = 2;
+    L.ty = pick_ty_cells((double)h_cells(0));
+    fcycle_down(who, 0);
+    coarse(who, 1, 0);
+    fcycle_up(who, 0);
+    if (h.cur[0] != 0) fprintf(stderr, "engine: hierarchy program parity\n");
+  }
+
   // Defect-correction solve, core/gmg/hierarchy.py:154-192 (solve): the
   // FP64 plane psi(h) (pool P, or the T pool of an FP64 batch when psi_q)
   // against the right-hand side rhs(h): rhs_flag 16 an FP64 plane (pool P),
@@ -3541,59 +3644,7 @@ struct Builder {
     };
     resid_norm(0, 0);
     for (int it = 0; it < maxite; it++) {
-      // F-cycle: b restricted down the fine levels (b0 -> b1 came with the
-      // residual), coarse tail, then V-cycles from each fine level upward.
-      // Level l = nfine - 1 - dd of an instance goes to l + 1 at
-      // bottom-aligned step dd; steps dd and dd - 1 share a k_restrict_b2
-      // launch (one-level launches where the program's mid-level phases
-      // are merged into persistent launches)
-      int Dmax = 0;
-      for (int i : who) Dmax = std::max(Dmax, b.H[i].d.nfine - 1);
-      for (int dd = Dmax - 1; dd >= 0; dd -= (b.persist > 0 ? 1 : 2)) {
-        if (b.persist > 0) {
-          double cells = 0.;
-          for (int i : who) {
-            const int l = b.H[i].d.nfine - 1 - dd;
-            if (l >= 1) cells += (double)(b.H[i].d.L[l].m - 2 * NH) * (b.H[i].d.L[l].n - 2 * NH);
-          }
-          const int ty = pick_ty_cells(cells);
-          std::vector<Task> rs;
-          for (int i : who) {
-            const int l = b.H[i].d.nfine - 1 - dd;
-            if (l >= 1) rr_tasks(i, l, 0, -1, -1, rs, ty / 2);
-          }
-          if (!rs.empty()) {
-            Launch& L = add(L_RR, rs);
-            L.flags = 2;
-            L.pred = 1;
-            L.ty = ty;
-          }
-          continue;
-        }
-        // output tiles of 8 rows, or of RB2_TY_SMALL rows where 8 would give
-        // at most RB2_TILES tiles (latency-bound launches: more, shorter tiles)
-        std::vector<Task> rs;
-        int rty = 8;
-        for (int ty : {8, RB2_TY_SMALL}) {
-          rs.clear();
-          rty = ty;
-          for (int i : who) {
-            const int l = b.H[i].d.nfine - 1 - dd;
-            if (dd >= 1 && l >= 1)
-              rb_tasks(i, l, 2, rs, ty);
-            else if (dd >= 1 && l == 0)
-              rb_tasks(i, 1, 1, rs, ty);
-            else if (dd == 0 && l >= 1)
-              rb_tasks(i, l, 1, rs, ty);
-          }
-          if (ty == 8 && (int)rs.size() > RB2_TILES) break;
-        }
-        if (!rs.empty()) {
-          Launch& L = add(L_RB2, rs);
-          L.pred = 1;
-          L.ty = rty;
-        }
-      }
+      fcycle_down(who, 1);
       coarse(who, 1, 1);
       // x0 += x (hierarchy.py:171) is folded into each instance's last
       // smoothing of the finest level (the up-leg of its V-cycle from level
@@ -3608,15 +3659,7 @@ struct Builder {
       upd_q = psi_q;
       if (fold_up)
         for (int i : who) upd_plane[i] = psi(b.H[i]);
-      for (int dd = 0; dd <= Dmax; dd++) {
-        std::vector<int> sub, st(b.ninst, 0);
-        for (int i : who)
-          if (b.H[i].d.nfine - 1 >= dd) {
-            sub.push_back(i);
-            st[i] = b.H[i].d.nfine - 1 - dd;
-          }
-        vcycle(sub, st, 3, 1, false);
-      }
+      fcycle_up(who, 1);
       upd_plane.clear();
       if (!fold_up) {
         std::vector<Task> up;
@@ -4278,9 +4321,11 @@ static void batch_free(Batch* b) {
   if (b->s) (void)hipStreamSynchronize(b->s);
   if (b->gexec) (void)hipGraphExecDestroy(b->gexec);
   if (b->graph) (void)hipGraphDestroy(b->graph);
-  if (b->P) (void)hipFree(b->P);
-  if (b->Q) (void)hipFree(b->Q);
-  if (b->B) (void)hipFree(b->B);
+  if (!b->hierarchy) {
+    if (b->P) (void)hipFree(b->P);
+    if (b->Q) (void)hipFree(b->Q);
+    if (b->B) (void)hipFree(b->B);
+  }
   if (b->dI) (void)hipFree(b->dI);
   if (b->dC) (void)hipFree(b->dC);
   if (b->dPk) (void)hipFree(b->dPk);
@@ -4365,6 +4410,7 @@ static int merge_persistent(Batch& b, std::vector<Launch>& prog) {
   return F2D_OK;
 }
 
+static int upload_programs(Batch& b);
 static int build_programs(Batch& b) {
   b.tasks.clear();
   b.spans.clear();
@@ -4374,6 +4420,10 @@ static int build_programs(Batch& b) {
   Builder bd(b);
   bd.lo = 0;
   bd.hi = b.ninst;
+  if (b.hierarchy) {
+    bd.hierarchy_programs();
+    return upload_programs(b);
+  }
   bd.prog = &b.prog_init;
   // initial inversion of every instance's state + diagnostics.  Euler and
   // Boussinesq both start from set_psi_from_vorticity (a full solve).
@@ -4415,6 +4465,11 @@ static int build_programs(Batch& b) {
   ETRY(merge_persistent(b, b.prog_diag));
   for (auto& po : b.prog_one) ETRY(merge_persistent(b, po));
   for (auto& po : b.prog_mom) ETRY(merge_persistent(b, po));
+  return upload_programs(b);
+}
+
+// the task tables and reduction scratch of the built programs
+static int upload_programs(Batch& b) {
   size_t np = 0;
   std::vector<const std::vector<Launch>*> progs = {&b.prog_init, &b.prog_step, &b.prog_diag};
   for (const auto& po : b.prog_one) progs.push_back(&po);
@@ -4487,7 +4542,9 @@ static int build_programs(Batch& b) {
     ECHK(hipMalloc(&b.fault, sizeof(int)));
     ECHK(hipMemset(b.fault, 0, sizeof(int)));
   }
-  ECHK(hipMemcpy(b.dS, b.spans.data(), b.spans.size() * sizeof(FoldSpan), hipMemcpyHostToDevice));
+  if (!b.spans.empty())
+    ECHK(hipMemcpy(b.dS, b.spans.data(), b.spans.size() * sizeof(FoldSpan),
+                   hipMemcpyHostToDevice));
   if (!b.slots.empty())
     ECHK(hipMemcpy(b.dSlot, b.slots.data(), b.slots.size() * sizeof(int), hipMemcpyHostToDevice));
   return F2D_OK;
@@ -4641,6 +4698,122 @@ static int apply_tuning(Batch& b, const f2d_batch_tuning* t) {
   return build_programs(b);
 }
 
+// ---- the launch programs of a stand-alone hierarchy (f2d_gmg) --------------
+// One instance whose levels are the caller's arrays: the engine's fused
+// kernels address them as offsets from the operator and the stencil bits of
+// level 0.  Both programs are captured graphs on those arrays, replayed on
+// the caller's stream.  Launched routine by routine from the host (about
+// 2000 launches of 3.7 us per solve) a 512^2 closed solve took 7.4 ms, a
+// 1024 x 512 twoVcycle 0.56 ms; so 0.91 and 0.17 ms.
+struct Hierarchy {
+  Batch b;
+  hipGraph_t graph[2] = {nullptr, nullptr};
+  hipGraphExec_t exec[2] = {nullptr, nullptr};
+};
+
+static void hierarchy_free(Hierarchy* h) {
+  if (!h) return;
+  (void)hipDeviceSynchronize();  // a launch may be in flight on the caller's stream
+  for (int k = 0; k < 2; k++) {
+    if (h->exec[k]) (void)hipGraphExecDestroy(h->exec[k]);
+    if (h->graph[k]) (void)hipGraphDestroy(h->graph[k]);
+  }
+  Batch* b = new Batch(std::move(h->b));
+  delete h;
+  batch_free(b);
+}
+
+static int hierarchy_build(Hierarchy& H, int nlev, const HierLevel* L, const uint8_t* bits,
+                           const double* w0, double omega) {
+  Batch& b = H.b;
+  b.hierarchy = true;
+  b.ninst = 1;
+  b.Q = L[0].A;
+  b.B = (int8_t*)bits;
+  b.H.resize(1);
+  HostInst& h = b.H[0];
+  InstD& d = h.d;
+  memset(&d, 0, sizeof d);
+  auto q = [&](const double* p) { return (long long)(p - (const double*)b.Q); };
+  auto y = [&](const int8_t* p) { return (long long)(p - b.B); };
+  d.nlev = nlev;
+  d.m = L[0].m;
+  d.n = L[0].n;
+  d.omega = omega;
+  for (int k = 0; k < 3; k++) d.kp[k] = -1;
+  d.msk = d.mskp = y(L[0].msk);
+  d.sb0 = 0;
+  d.a0fly = 1;
+  for (int k = 0; k < 5; k++) d.w0[k] = w0[k];
+  std::vector<int8_t> msk((size_t)d.m * d.n);
+  ECHK(hipMemcpy(msk.data(), L[0].msk, msk.size(), hipMemcpyDeviceToHost));
+  h.count_solid(msk.data(), d.m, d.n);
+  for (int l = 0; l < nlev; l++) {
+    LevD& G = d.L[l];
+    G.m = L[l].m;
+    G.n = L[l].n;
+    G.A = q(L[l].A);
+    G.b = q(L[l].b);
+    G.x[0] = q(L[l].x);
+    G.x[1] = q(L[l].t);
+    G.msk = y(L[l].msk);
+    h.buf[l][0] = G.x[0];
+    h.buf[l][1] = G.x[1];
+    h.cur[l] = 0;
+    const size_t S = (size_t)G.m * G.n;
+    if (l > 0 && S <= COARSE_CELLS) {
+      h.cA[l].resize(5 * S);
+      h.cM[l].resize(S);
+      ECHK(hipMemcpy(h.cA[l].data(), L[l].A, 5 * S * sizeof(double), hipMemcpyDeviceToHost));
+      ECHK(hipMemcpy(h.cM[l].data(), L[l].msk, S, hipMemcpyDeviceToHost));
+    }
+  }
+  int k0 = 0;
+  ETRY(first_coarse_level(d, lds_budget(0), sizeof(double), &k0));
+  d.nfine = k0;
+  h.coarse_lds = coarse_bytes(d, k0, sizeof(double));
+  ECHK(hipMalloc(&b.dI, sizeof(InstD)));
+  ECHK(hipMalloc(&b.dD, sizeof(DynD)));
+  DynD dyn;
+  memset(&dyn, 0, sizeof dyn);
+  dyn.run = dyn.active = 1;
+  ECHK(hipMemcpy(b.dD, &dyn, sizeof dyn, hipMemcpyHostToDevice));
+  // the launch shapes the autotuner picks for one grid
+  const f2d_batch_tuning t{0, 1024, 0, 0};
+  ETRY(apply_tuning(b, &t));
+  ECHK(hipStreamCreateWithFlags(&b.s, hipStreamNonBlocking));
+  return F2D_OK;
+}
+
+int hierarchy_create(int nlev, const HierLevel* L, const uint8_t* bits, const double* w0,
+                     double omega, Hierarchy** out) {
+  *out = nullptr;
+  // what the fused kernels take: at least two levels, arrays below 4 GiB
+  if (nlev < 2 || nlev > MAXLEV || (double)L[0].m * L[0].n * 40. >= 4294967296.) return F2D_OK;
+  Hierarchy* H = new Hierarchy();
+  const int rc = hierarchy_build(*H, nlev, L, bits, w0, omega);
+  if (rc) {
+    hierarchy_free(H);
+    return rc;
+  }
+  *out = H;
+  return F2D_OK;
+}
+int hierarchy_run(Hierarchy* h, int which, hipStream_t s) {
+  if (!h->exec[which]) {  // captured by the first call that needs it
+    ECHK(hipStreamBeginCapture(h->b.s, hipStreamCaptureModeThreadLocal));
+    const int rc = run_prog(h->b, which == 0 ? h->b.prog_step : h->b.prog_init);
+    const hipError_t e = hipStreamEndCapture(h->b.s, &h->graph[which]);
+    if (rc) return rc;
+    ECHK(e);
+    ECHK(hipGraphInstantiate(&h->exec[which], h->graph[which], nullptr, nullptr, 0));
+  }
+  ECHK(hipGraphLaunch(h->exec[which], s));
+  return F2D_OK;
+}
+void hierarchy_destroy(Hierarchy* h) { hierarchy_free(h); }
+const char* hierarchy_error() { return e_err.c_str(); }
+
 }  // namespace eng
 }  // namespace f2d
 
@@ -4697,7 +4870,7 @@ int f2d_batch_create(int ninst, const f2d_model_params* params, const int8_t* co
     const f2d_model_params& p = params[i];
     HostInst& h = b->H[i];
     h.p = p;
-    h.hmsk.assign(msks[i], msks[i] + (size_t)(p.ny + 2 * NH) * (p.nx + 2 * NH));
+    h.count_solid(msks[i], p.ny + 2 * NH, p.nx + 2 * NH);
     InstD& d = h.d;
     memset(&d, 0, sizeof d);
     if (p.model != 0 && p.model != 1) return bail(efail(F2D_E_ARG, "model"));

@@ -407,6 +407,17 @@ __global__ void k_afinest(const int8_t* __restrict__ msk, double* __restrict__ A
   }
 }
 
+// Stencil bits of the level-0 operator (five planes): bit k (k < 4) where
+// coupling A_k is nonzero, bit 4 the cell mask.
+__global__ void k_stencil_bits(const int8_t* __restrict__ msk, const double* __restrict__ A,
+                               uint8_t* __restrict__ bits, size_t cnt) {
+  const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= cnt) return;
+  unsigned b = msk[q] != 0 ? 16u : 0u;
+  for (int k = 0; k < 4; k++) b |= A[k * cnt + q] != 0. ? 1u << k : 0u;
+  bits[q] = (uint8_t)b;
+}
+
 // Corner mask (core/operators.py:59-67): 1 where celltocorner(msk) == 1.
 __global__ void k_corner_mask(const int8_t* __restrict__ msk, int8_t* __restrict__ mskp, int m,
                               int n) {
@@ -928,6 +939,11 @@ __global__ void k_helmholtz_shift(double* __restrict__ A5, size_t cnt, double sh
 }
 void launch_helmholtz_shift(double* A5, size_t cnt, double shift, hipStream_t s) {
   hipLaunchKernelGGL(k_helmholtz_shift, grid1(cnt), B1, 0, s, A5, cnt, shift);
+}
+void launch_stencil_bits(const int8_t* msk, const double* A, uint8_t* bits, int m, int n,
+                         hipStream_t s) {
+  const size_t cnt = (size_t)m * n;
+  hipLaunchKernelGGL(k_stencil_bits, grid1(cnt), B1, 0, s, msk, A, bits, cnt);
 }
 void launch_corner_mask(const int8_t* msk, int8_t* mskp, int m, int n, hipStream_t s) {
   hipLaunchKernelGGL(k_corner_mask, grid2(n, m), B2, 0, s, msk, mskp, m, n);

@@ -4,7 +4,9 @@
 // The cycle logic restates core/gmg/hierarchy.py (Vcycle, Fcycle, solve,
 // twoVcycle) and the model logic core/operators.py, core/timescheme.py,
 // core/euler.py and core/boussinesq.py; every arithmetic step is a kernel
-// from f2d_ops.hip on device-resident buffers.  The only host round trips
+// from f2d_ops.hip on device-resident buffers, except the cycles of solve and
+// twoVcycle, which replay the engine's fused kernels (eng::Hierarchy) on the
+// hierarchy's arrays.  The only host round trips
 // are the residual norms that decide the solve loop (hierarchy.py:169) and
 // the diagnostics that feed cst[3] (fluid2d.py:397).
 #include <math.h>
@@ -17,6 +19,7 @@
 #include <vector>
 
 #include "../../include/fluid2d_amd.h"
+#include "f2d_engine.h"
 #include "f2d_ops.h"
 
 using namespace f2d;
@@ -98,10 +101,17 @@ struct f2d_gmg {
   double* scal = nullptr;     // device scalars
   double* hscal = nullptr;    // pinned host mirror
   hipStream_t s = nullptr;
+  double w0[5] = {0., 0., 0., 0., 0.};  // level-0 operator: weights, and its
+  uint8_t* bits = nullptr;              // stencil bits
+  // the cycles of solve and twoVcycle on the engine's fused kernels; null:
+  // one launch per routine
+  eng::Hierarchy* fused = nullptr;
 };
 
 static int gmg_free(f2d_gmg* g) {
   if (!g) return F2D_OK;
+  eng::hierarchy_destroy(g->fused);
+  dfree(g->bits);
   for (int l = 0; l < g->nlev; l++) {
     Level& L = g->L[l];
     dfree(L.msk);
@@ -158,7 +168,9 @@ static int gmg_build(int nx, int ny, double dx, double dy, double hydroepsilon, 
     L.m = lv[l].first;
     L.n = lv[l].second;
     const size_t sz = L.size();
-    if ((rc = dalloc(&L.msk, sz)) || (rc = dalloc(&L.A, 5 * sz)) || (rc = dalloc(&L.x, sz)) ||
+    // (256 bytes of slack: the generic coarse kernel's 16-byte LDS loads
+    // round the tails of operator and mask up)
+    if ((rc = dalloc(&L.msk, sz + 256)) || (rc = dalloc(&L.A, 5 * sz + 32)) || (rc = dalloc(&L.x, sz)) ||
         (rc = dalloc(&L.b, sz)) || (rc = dalloc(&L.r, sz)) || (rc = dalloc(&L.t, sz)))
       return bail(rc);
     if (hipMemset(L.x, 0, sz * 8) || hipMemset(L.b, 0, sz * 8) || hipMemset(L.r, 0, sz * 8) ||
@@ -197,6 +209,7 @@ static int gmg_build(int nx, int ny, double dx, double dy, double hydroepsilon, 
       memcpy(st.w, w, sizeof w);
     }
     launch_afinest(L.msk, A9[0], st, 1. / (dx * dy), L.m, L.n, s);
+    for (int k = 0; k < 5; k++) g->w0[k] = st.w[k] * (1. / (dx * dy)) * 1. * 1.;
   }
   for (int l = 1; l < g->nlev; l++) {
     Level &F = g->L[l - 1], &C = g->L[l];
@@ -215,6 +228,26 @@ static int gmg_build(int nx, int ny, double dx, double dy, double hydroepsilon, 
   if (e != hipSuccess) return bail(fail(F2D_E_HIP, "gmg setup: %s", hipGetErrorString(e)));
   *out = g;
   return F2D_OK;
+}
+
+// (Re)builds the fused cycles of a hierarchy from its operators.  Every
+// value of a level-0 plane is its weight or 0 by construction (launch_afinest;
+// the Helmholtz shift changes every nonzero centre alike).
+static int gmg_fuse(f2d_gmg* g) {
+  eng::hierarchy_destroy(g->fused);
+  g->fused = nullptr;
+  const Level& L0 = g->L[0];
+  if (!g->bits) TRY(dalloc(&g->bits, L0.size()));
+  launch_stencil_bits(L0.msk, L0.A, g->bits, L0.m, L0.n, g->s);
+  LAUNCHCHK();
+  HIPCHK(hipStreamSynchronize(g->s));
+  std::vector<eng::HierLevel> v(g->nlev);
+  for (int l = 0; l < g->nlev; l++) {
+    const Level& L = g->L[l];
+    v[l] = eng::HierLevel{L.m, L.n, L.msk, L.A, L.x, L.b, L.t};
+  }
+  const int rc = eng::hierarchy_create(g->nlev, v.data(), g->bits, g->w0, g->omega, &g->fused);
+  return rc ? fail(rc, "%s", eng::hierarchy_error()) : F2D_OK;
 }
 
 // core/gmg/level.py:340-368 (smooth nite times, fill after each)
@@ -293,7 +326,12 @@ static int g_solve(f2d_gmg* g, double* x, const double* b, int maxite, double to
   double res0 = nb0 / normeb, res = res0;
   int nite = 0, ndiv = 0;
   while (nite < maxite && res0 > tol) {
-    g_fcycle(g, 0);
+    if (g->fused) {
+      const int rc = eng::hierarchy_run(g->fused, 1, g->s);
+      if (rc) return fail(rc, "%s", eng::hierarchy_error());
+    } else {
+      g_fcycle(g, 0);
+    }
     launch_add_inplace(x, (const double*)L0.x, L0.size(), g->s);
     g_residual(g, 0, x, b, L0.b);
     double nb;
@@ -316,12 +354,18 @@ static int g_solve(f2d_gmg* g, double* x, const double* b, int maxite, double to
 
 // core/gmg/hierarchy.py:207-218 (the residual at the top of each cycle is
 // overwritten by Vcycle before it is read, so it is not recomputed)
-static void g_twovcycle(f2d_gmg* g, double* x, const double* b) {
+static int g_twovcycle(f2d_gmg* g, double* x, const double* b) {
   Level& L0 = g->L[0];
   launch_copy(L0.x, (const double*)x, L0.size(), g->s);
   launch_copy(L0.b, b, L0.size(), g->s);
-  for (int k = 0; k < 2; k++) g_vcycle(g, 0);
+  if (g->fused) {
+    const int rc = eng::hierarchy_run(g->fused, 0, g->s);
+    if (rc) return fail(rc, "%s", eng::hierarchy_error());
+  } else {
+    for (int k = 0; k < 2; k++) g_vcycle(g, 0);
+  }
   launch_copy(x, (const double*)L0.x, L0.size(), g->s);
+  return F2D_OK;
 }
 
 // ---------------------------------------------------------------------------
@@ -436,7 +480,7 @@ static int invert_vorticity(f2d_model* M, double* x, bool full, bool island = fa
   launch_celltocorner(M->F(x, I_VORT), M->work, M->m, M->n, M->s);
   if (island) launch_sub_inplace(M->work, M->rhsp, M->fsz, M->s);
   if (!full) {
-    g_twovcycle(M->gmg, psi, M->work);
+    TRY(g_twovcycle(M->gmg, psi, M->work));
   } else {
     int nite = 0;
     double res = 0.;
@@ -941,7 +985,13 @@ int f2d_domain_sum_f64_noalloc(const double* x, int nh, int m, int n, double* ou
 int f2d_gmg_create(int nx, int ny, int nh, double dx, double dy, double hydroepsilon, double omega,
                    const int8_t* mskp_host, f2d_gmg** out) {
   if (nh != NH) return fail(F2D_E_ARG, "nh must be 3");
-  return gmg_build(nx, ny, dx, dy, hydroepsilon, omega, mskp_host, out);
+  TRY(gmg_build(nx, ny, dx, dy, hydroepsilon, omega, mskp_host, out));
+  const int rc = gmg_fuse(*out);
+  if (rc) {
+    gmg_free(*out);
+    *out = nullptr;
+  }
+  return rc;
 }
 int f2d_gmg_destroy(f2d_gmg* g) { return gmg_free(g); }
 int f2d_gmg_set_helmholtz(f2d_gmg* g, double Rd) {
@@ -951,7 +1001,8 @@ int f2d_gmg_set_helmholtz(f2d_gmg* g, double Rd) {
     launch_helmholtz_shift(g->L[l].A + 4 * g->L[l].size(), g->L[l].size(), shift, g->s);
   LAUNCHCHK();
   HIPCHK(hipStreamSynchronize(g->s));
-  return F2D_OK;
+  g->w0[4] -= shift;
+  return gmg_fuse(g);
 }
 int f2d_gmg_nlevels(const f2d_gmg* g, int* nlev) {
   *nlev = g->nlev;
@@ -989,7 +1040,7 @@ int f2d_gmg_fcycle(f2d_gmg* g, int lev1) {
   return F2D_OK;
 }
 int f2d_gmg_twovcycle(f2d_gmg* g, double* x, const double* b) {
-  g_twovcycle(g, x, b);
+  TRY(g_twovcycle(g, x, b));
   LAUNCHCHK();
   HIPCHK(hipStreamSynchronize(g->s));
   return F2D_OK;
@@ -1054,7 +1105,8 @@ int f2d_model_create(const f2d_model_params* p, const int8_t* msk_host, f2d_mode
   if (hipMemcpy(mskp.data(), M->mskp, M->fsz, hipMemcpyDeviceToHost) != hipSuccess)
     return bail(fail(F2D_E_HIP, "download corner mask"));
   if ((rc = gmg_build(p->nx, p->ny, M->dx, M->dy, p->hydroepsilon, 8. / 9., mskp.data(),
-                      &M->gmg)))
+                      &M->gmg)) ||
+      (rc = gmg_fuse(M->gmg)))
     return bail(rc);
   M->cst[0] = M->dx;
   M->cst[1] = M->dy;

@@ -3,7 +3,8 @@
 ``Gmg(param, mskp)`` builds the level hierarchy, masks and operators on the
 GPU (core/gmg/hierarchy.py:23-84, core/gmg/level.py:24-335) and exposes the
 reference's cycle methods.  Arrays passed to ``solve`` / ``twoVcycle`` are
-device arrays of the finest level's shape.
+device arrays of the finest level's shape; both use the level arrays as
+scratch (``Vcycle`` and ``Fcycle`` leave each level's x and b in them).
 """
 import ctypes as C
 
