@@ -20,15 +20,16 @@ struct UpParams {
   int method, order;
 };
 
-template <typename T>
+// LC: method 2 (log-cosh) may occur.  Its log and cosh, inlined at every
+// edge, are most of a kernel's code; callers that never see it leave it out.
+template <bool LC = true, typename T>
 __device__ __forceinline__ T split_speed(T vel, const UpParams<T>& p) {
-  T UU = T(0);
-  if (p.method == 0) UU = fabs(vel);
+  T UU = fabs(vel);
   if (p.method == 1) {
-    UU = fabs(vel);
     if (UU < p.u1) UU = p.aa * (vel * vel) + p.bb;
   }
-  if (p.method == 2) UU = T(2) * p.KK + log(cosh(vel * p.a)) / p.a;
+  if constexpr (LC)
+    if (p.method == 2) UU = T(2) * p.KK + log(cosh(vel * p.a)) / p.a;
   return UU;
 }
 
@@ -36,16 +37,23 @@ __device__ __forceinline__ T split_speed(T vel, const UpParams<T>& p) {
 // mk[-2s..3s], values q[-2s..3s], edge velocity vel.
 // core/fortran_advection.f90:73-146.  Generic over the value accessor Q
 // (Q(k) returns the tracer at offset k*s) so stage states can be formed on
-// the fly.
-template <typename T, typename Q>
+// the fly.  FULL5: the whole window is fluid and the order is 5 (no mask is
+// read).
+template <bool FULL5 = false, bool LC = true, typename T, typename Q>
 __device__ __forceinline__ T up_edge_flux_q(const int8_t* mk, ptrdiff_t s, T vel,
                                             const UpParams<T>& p, Q q) {
-  if (mk[0] + mk[s] != 2) return T(0);
+  if constexpr (!FULL5)
+    if (mk[0] + mk[s] != 2) return T(0);
   const T d1 = T(W32(1, 30)), d2 = T(-W32(13, 60)), d3 = T(W32(47, 60)), d4 = T(W32(9, 20)),
           d5 = T(-W32(1, 20));
   const T c1 = T(-W32(1, 6)), c2 = T(W32(5, 6)), c3 = T(W32(2, 6));
-  const T UU = split_speed(vel, p);
+  const T UU = split_speed<LC>(vel, p);
   const T up = T(0.5) * (vel + UU), um = T(0.5) * (vel - UU);
+  if constexpr (FULL5) {
+    const T qp = d1 * q(-2) + d2 * q(-1) + d3 * q(0) + d4 * q(1) + d5 * q(2);
+    const T qm = d5 * q(-1) + d4 * q(0) + d3 * q(1) + d2 * q(2) + d1 * q(3);
+    return up * qp + um * qm;
+  }
   const int m_2 = mk[-2 * s], m_1 = mk[-s], m0 = mk[0], m1 = mk[s], m2 = mk[2 * s],
             m3 = mk[3 * s];
   const int s5p = m_2 + m_1 + m0 + m1 + m2, s3p = m_1 + m0 + m1;

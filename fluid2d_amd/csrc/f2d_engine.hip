@@ -158,16 +158,32 @@ struct TrVal {
   int8_t m;
 };
 
-// NTR: tracers advected (1 Euler, 2 Boussinesq); each launch holds instances
-// of one model
-template <typename T, int NTR>
+// NTR: tracers advected (1 Euler, 2 Boussinesq); UP: upwind (odd) orders;
+// each launch holds instances of one model and one kind of order.
+//
+// What bounds it: vector instructions.  A thread owns a strip of four rows of
+// one column: the x-edges on their left and the y-edges below them, each
+// with its velocity in a register (only tracers and mask pass through LDS), the
+// y-edges sharing their tracer window; what a cell needs of its neighbours'
+// fluxes comes by lane shuffles (x) and one LDS row per strip (y).  A tile
+// whose tracer window is all fluid takes the fifth-order flux without masks
+// (the general form reads six masks per edge and holds every order).  The
+// log-cosh splitting, which no instance can have, is not compiled in: inlined
+// at every edge it made the kernel 13.9 k instructions long (now 7.6 k).
+// Mean of the three stages: 2048 x 1024 two tracers 72.8 -> 46.9 us (3.6 TB/s
+// of stage state and tendencies), 1024^2 one tracer 20.9 -> 17.1 us (the last
+// stage 5 TB/s), 128^2 12.2 -> 7.1 us, 32 mixed instances of 64^2..512^2 49.1
+// -> 36.4 us.
+template <typename T, int NTR, bool UP>
 __global__ void __launch_bounds__(256) k_rhs(const Task* __restrict__ tasks,
                                              const InstD* __restrict__ I, double* P, T* Q,
                                              const int8_t* __restrict__ B,
                                              const DynD* __restrict__ dyn, int stage, int out_k) {
+  constexpr int RS = 4;  // rows of a strip
+  static_assert(TY == 4 * RS && TX == 64, "one wavefront per strip row");
   __shared__ double qs[NTR][QH * QW];
-  __shared__ double us[TY * (TX + 1)];
-  __shared__ double vs[(TY + 1) * TX];
+  __shared__ double fxe[NTR][TY];                // x-edge right of the last column
+  __shared__ double fys[NTR][TY / RS + 1][TX];  // y-edge below each strip's first row, and the top
   __shared__ int8_t ms[QH * QW];
   const int ti = task_index();
   const Task tk = tasks[ti];
@@ -192,12 +208,16 @@ __global__ void __launch_bounds__(256) k_rhs(const Task* __restrict__ tasks,
     S.c = stage == 1 ? dt / 3. : 0.5 * dt;
   }
   const int8_t* msk = B + in.msk;
-  const int tid = threadIdx.y * blockDim.x + threadIdx.x, nt = blockDim.x * blockDim.y;
-  const int y0 = tk.y0, x0 = tk.x0;
-  // tiles: tracer rows [y0-3, y0+TY+2] x cols [x0-3, x0+TX+2]; each tile's
-  // loads are issued together (compile-time trip counts, clamped in-bounds
-  // addresses), then stored
-  (void)nt;
+  const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * 64 + tx;
+  const int y0 = tk.y0, x0 = tk.x0, r0 = ty * RS;
+  // the strip's edge velocities, and one edge more: the first wavefront the
+  // y-edges above the tile, 16 lanes of the second the x-edges right of it
+  const int er = ty == 0 ? TY : (ty == 1 && tx < TY ? tx : -1);
+  double uv[RS], vv[RS], ev = 0.;
+  bool full = true;
+  // tiles: tracer rows [y0-3, y0+TY+2] x cols [x0-3, x0+TX+2]; the loads are
+  // issued together (compile-time trip counts, clamped in-bounds addresses),
+  // then stored
   auto load_tiles = [&](auto kind) {
     constexpr int K = decltype(kind)::value;
     tile_load<(QH * QW + 255) / 256>(tid, QH * QW, [&](int q) {
@@ -216,140 +236,141 @@ __global__ void __launch_bounds__(256) k_rhs(const Task* __restrict__ tasks,
       return v;
     }, [&](int q, const TrVal& v) {
       ms[q] = v.m;
+      full = full && v.m == 1;
       qs[0][q] = v.q0;
       if constexpr (NTR > 1) qs[NTR - 1][q] = v.q1;
     });
-    tile_load<(TY * (TX + 1) + 255) / 256>(tid, TY * (TX + 1), [&](int q) {
-      const int r = q / (TX + 1), c = q - r * (TX + 1);  // u on rows y0.., cols x0-1..
-      const int j = y0 + r, i = x0 - 1 + c;
+    auto vel = [&](int f, int j, int i) {
       const bool ok = j < m && i < n;
-      const double v = S.template at<K>((uint32_t)(2 * F) + (ok ? at32(j, i, n) : 0u));
+      const double v = S.template at<K>((uint32_t)(f * F) + (ok ? at32(j, i, n) : 0u));
       return ok ? v : 0.;
-    }, [&](int q, double v) { us[q] = v; });
-    tile_load<((TY + 1) * TX + 255) / 256>(tid, (TY + 1) * TX, [&](int q) {
-      const int r = q / TX, c = q - r * TX;  // v on rows y0-1.., cols x0..
-      const int j = y0 - 1 + r, i = x0 + c;
-      const bool ok = j < m && i < n;
-      const double v = S.template at<K>((uint32_t)(3 * F) + (ok ? at32(j, i, n) : 0u));
-      return ok ? v : 0.;
-    }, [&](int q, double v) { vs[q] = v; });
-  };
-  auto by_kind = [&]() {
-    switch (S.kind) {
-      case 0: load_tiles(std::integral_constant<int, 0>()); break;
-      case 1: load_tiles(std::integral_constant<int, 1>()); break;
-      case 2: load_tiles(std::integral_constant<int, 2>()); break;
-      default: load_tiles(std::integral_constant<int, 3>()); break;
+    };
+#pragma unroll
+    for (int k = 0; k < RS; k++) {
+      uv[k] = vel(2, y0 + r0 + k, x0 - 1 + tx);
+      vv[k] = vel(3, y0 - 1 + r0 + k, x0 + tx);
     }
+    if (er >= 0)
+      ev = ty == 0 ? vel(3, y0 - 1 + TY, x0 + tx) : vel(2, y0 + er, x0 - 1 + TX);
   };
-  by_kind();
-  __syncthreads();
+  switch (S.kind) {
+    case 0: load_tiles(std::integral_constant<int, 0>()); break;
+    case 1: load_tiles(std::integral_constant<int, 1>()); break;
+    case 2: load_tiles(std::integral_constant<int, 2>()); break;
+    default: load_tiles(std::integral_constant<int, 3>()); break;
+  }
+  full = block_all4(full) != 0;  // (the tiles' barrier)
   // advection parameters (core/fortran_advection.f90:46-60), cst[3] = umax
   UpParams<double> p;
-  const double umax = d.umax, logcosh = 0.05;
   p.zdx = 1. / in.dx;
   p.zdy = 1. / in.dy;
   {
-    const double a = logcosh / umax;
-    p.a = a;
-    p.KK = (umax - log(cosh(umax * a)) / a) * 0.5;
-    const double u1 = in.aparab * umax;
+    const double u1 = in.aparab * d.umax;
     p.u1 = u1;
     p.aa = 1. / (2. * u1);
     p.bb = u1 * 0.5;
   }
+  p.a = p.KK = 0.;
   p.method = in.method;
   p.order = in.order;
   UpParams<T> pt;
   pt.zdx = T(p.zdx);
   pt.zdy = T(p.zdy);
-  pt.a = T(p.a);
-  pt.KK = T(p.KK);
+  pt.a = pt.KK = T(0);
   pt.u1 = T(p.u1);
   pt.aa = T(p.aa);
   pt.bb = T(p.bb);
   pt.method = p.method;
   pt.order = p.order;
-  const bool upwind = in.order % 2 == 1;
   const bool kforce = stage == (in.tscheme == 0 ? 2 : 0);
   T* out = Q + in.k[out_k];
   constexpr bool MIXED = sizeof(T) == 4;
-  // Edge fluxes, each computed once: fx[r][e] on the x-edge between tile
-  // cells (r, e-1) and (r, e), fy[e][c] on the y-edge between (e-1, c) and
-  // (e, c).  FP64: the reference's flux arithmetic.  Mixed: the flux is
-  // linear in q, F(q) = F(q - q_L) + q_L F(1) with q_L the tracer of the
-  // edge's left (lower) cell: the first term in FP32 on differences taken
-  // in FP64, the unit-field flux F(1) and the sum in FP64, so the rounding
-  // scales with the local variation of q.
-  // Each edge's flux overwrites the edge velocity it was computed from (the
-  // same thread reads and writes the same slot; with two tracers the thread
-  // keeps its edges' velocities in registers for the second), so the tile
-  // needs no flux arrays of its own: four workgroups per CU with one tracer,
-  // three with two.
-  double(*fx)[TX + 1] = (double(*)[TX + 1])us;
-  double(*fy)[TX] = (double(*)[TX])vs;
-  constexpr int KU = (TY * (TX + 1) + 255) / 256, KV = ((TY + 1) * TX + 255) / 256;
-  double uvel[NTR > 1 ? KU : 1], vvel[NTR > 1 ? KV : 1];
-  (void)uvel;
-  (void)vvel;
-  auto edge_flux = [&](const double* qt, int lq, ptrdiff_t st, double vel) -> double {
-    const double ql = MIXED ? qt[lq] : 0.;
-    auto qv = [qt, lq, st, ql](int k) { return T(qt[lq + k * st] - ql); };
-    T f;
-    if (upwind)
-      f = up_edge_flux_q(ms + lq, st, T(vel), pt, qv);
-    else
-      f = ce_edge_flux_q(ms + lq, st, T(vel), in.order, true, qv);
-    if (!MIXED) return (double)f;
+  // FP64: the reference's flux arithmetic.  Mixed: the flux is linear in q,
+  // F(q) = F(q - q_L) + q_L F(1) with q_L the tracer of the edge's left
+  // (lower) cell: the first term in FP32 on differences taken in FP64, the
+  // unit-field flux F(1) and the sum in FP64, so the rounding scales with the
+  // local variation of q.  qa(k): the tracer at offset k from that cell.
+  auto edge_flux = [&](auto f5, const int8_t* mk, ptrdiff_t st, double vel, auto qa) -> double {
+    constexpr bool F5 = decltype(f5)::value;
+    const double ql = MIXED ? qa(0) : 0.;
+    auto qv = [&](int k) { return T(qa(k) - ql); };
     auto one = [](int) { return 1.; };
-    const double u1 = upwind ? up_edge_flux_q(ms + lq, st, vel, p, one)
-                             : ce_edge_flux_q(ms + lq, st, vel, in.order, true, one);
+    T f;
+    double u1 = 0.;
+    if constexpr (UP) {
+      f = up_edge_flux_q<F5, false>(mk, st, T(vel), pt, qv);
+      if constexpr (MIXED) u1 = up_edge_flux_q<F5, false>(mk, st, vel, p, one);
+    } else {
+      f = ce_edge_flux_q(mk, st, T(vel), in.order, true, qv);
+      if constexpr (MIXED) u1 = ce_edge_flux_q(mk, st, vel, in.order, true, one);
+    }
+    if (!MIXED) return (double)f;
     return (double)f + ql * u1;
   };
+  double fx[NTR][RS], fy[NTR][RS];
+  auto fluxes = [&](auto f5) {
+    constexpr bool F5 = decltype(f5)::value;
+#pragma unroll
+    for (int t = 0; t < NTR; t++) {
+      const double* qt = qs[t];
+      // x-edge left of tile cell (r, tx): its left cell is tile column tx + 2
+      auto xq = [&](int r, int c) {
+        const double* q = qt + (r + 3) * QW + c + 2;
+        return [q](int k) { return q[k]; };
+      };
+      // y-edge below tile cell (r, c): its lower cell is tile row r + 2
+      auto yq = [&](int r, int c) {
+        const double* q = qt + (r + 2) * QW + c + 3;
+        return [q](int k) { return q[k * QW]; };
+      };
+      auto xm = [&](int r, int c) { return ms + (r + 3) * QW + c + 2; };
+      auto ym = [&](int r, int c) { return ms + (r + 2) * QW + c + 3; };
+      if constexpr (F5) {
+        double w[RS + 5];  // the strip's window: tile rows r0 .. r0 + RS + 4
+#pragma unroll
+        for (int k = 0; k < RS + 5; k++) w[k] = qt[(r0 + k) * QW + tx + 3];
+#pragma unroll
+        for (int k = 0; k < RS; k++) {
+          fx[t][k] = edge_flux(f5, ms, 1, uv[k], xq(r0 + k, tx));
+          fy[t][k] = edge_flux(f5, ms, QW, vv[k], [&](int e) { return w[k + 2 + e]; });
+        }
+      } else {
+#pragma unroll
+        for (int k = 0; k < RS; k++) {
+          fx[t][k] = edge_flux(f5, xm(r0 + k, tx), 1, uv[k], xq(r0 + k, tx));
+          fy[t][k] = edge_flux(f5, ym(r0 + k, tx), QW, vv[k], yq(r0 + k, tx));
+        }
+      }
+      fys[t][ty][tx] = fy[t][0];
+      if (ty == 0)
+        fys[t][TY / RS][tx] = edge_flux(f5, ym(TY, tx), QW, ev, yq(TY, tx));
+      else if (er >= 0)
+        fxe[t][er] = edge_flux(f5, xm(er, TX), 1, ev, xq(er, TX));
+    }
+  };
+  const bool fast = UP && full && in.order == 5;
+  if (fast)
+    fluxes(std::true_type());
+  else
+    fluxes(std::false_type());
+  __syncthreads();
+  const bool diff = in.diffusion && kforce;
 #pragma unroll
   for (int t = 0; t < NTR; t++) {
     const double* qt = qs[t];
-    if (t > 0) __syncthreads();  // the previous tracer's divergence read fx, fy
-    if constexpr (NTR == 1) {
-      for (int q = tid; q < TY * (TX + 1); q += 256) {
-        const int r = q / (TX + 1), e = q - r * (TX + 1);
-        fx[r][e] = edge_flux(qt, (r + 3) * QW + e + 2, 1, us[q]);
-      }
-      for (int q = tid; q < (TY + 1) * TX; q += 256) {
-        const int e = q / TX, c = q - e * TX;
-        fy[e][c] = edge_flux(qt, (e + 2) * QW + c + 3, (ptrdiff_t)QW, vs[q]);
-      }
-    } else {
 #pragma unroll
-      for (int k = 0; k < KU; k++) {
-        const int q = tid + 256 * k;
-        if (q < TY * (TX + 1)) {
-          const int r = q / (TX + 1), e = q - r * (TX + 1);
-          if (t == 0) uvel[k] = us[q];
-          fx[r][e] = edge_flux(qt, (r + 3) * QW + e + 2, 1, uvel[k]);
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < KV; k++) {
-        const int q = tid + 256 * k;
-        if (q < (TY + 1) * TX) {
-          const int e = q / TX, c = q - e * TX;
-          if (t == 0) vvel[k] = vs[q];
-          fy[e][c] = edge_flux(qt, (e + 2) * QW + c + 3, (ptrdiff_t)QW, vvel[k]);
-        }
-      }
-    }
-    __syncthreads();
-    for (int r = threadIdx.y; r < TY; r += blockDim.y) {
-      const int J = y0 + r, Ic = x0 + threadIdx.x;
+    for (int k = 0; k < RS; k++) {
+      const int r = r0 + k, J = y0 + r, Ic = x0 + tx;
+      double fr = __shfl_down(fx[t][k], 1, 64);  // (before any lane leaves)
       if (J >= m - NH || Ic >= n - NH) continue;
-      const int lq = (r + 3) * QW + threadIdx.x + 3;  // cell in the tracer/mask tile
-      const int c = threadIdx.x;
+      if (tx == TX - 1) fr = fxe[t][r];
+      const double fu = k + 1 < RS ? fy[t][k + 1 < RS ? k + 1 : 0] : fys[t][ty + 1][tx];
+      const int lq = (r + 3) * QW + tx + 3;  // cell in the tracer/mask tile
       T val;
       if (MIXED)
-        val = T(-p.zdx * (fx[r][c + 1] - fx[r][c]) - p.zdy * (fy[r + 1][c] - fy[r][c]));
+        val = T(-p.zdx * (fr - fx[t][k]) - p.zdy * (fu - fy[t][k]));
       else
-        val = T(-pt.zdx * T(fx[r][c + 1] - fx[r][c]) - pt.zdy * T(fy[r + 1][c] - fy[r][c]));
+        val = T(-pt.zdx * T(fr - fx[t][k]) - pt.zdy * T(fu - fy[t][k]));
       const int8_t mc = ms[lq];
       if constexpr (NTR > 1) {
         if (t == 0) {  // Boussinesq: y *= msk; add_torque
@@ -362,7 +383,7 @@ __global__ void __launch_bounds__(256) k_rhs(const Task* __restrict__ tasks,
                             T(mc);
         }
       }
-      if (in.diffusion && kforce && mc == 1) {  // add_diffusion
+      if (diff && mc == 1) {  // add_diffusion
         const double coefd =
             (in.model == 0 ? 1. : (in.tscheme == 0 ? 1.5 : 1.)) * (t == 0 ? in.kd0 : in.kd1);
         const T coef = T(coefd / (in.dx * in.dx));
@@ -3894,18 +3915,20 @@ struct Builder {
     const bool ssp = b.H[0].d.tscheme == 0;
     const int kforcing = ssp ? 2 : 0;
     for (int stage = 0; stage < 3; stage++) {
-      // one advection launch per model (tracer count)
-      for (int model = 0; model < 2; model++) {
+      // one advection launch per model (tracer count) and kind of order
+      for (int kind = 0; kind < 4; kind++) {
+        const int model = kind & 1, up = kind < 2 ? 1 : 0;
         std::vector<Task> ts;
         for (int i : who) {
           HostInst& h = b.H[i];
-          if (h.d.model == model) tiles(ts, mk_task(i, 0, 0, 0), NH, h.d.m - NH, NH, h.d.n - NH);
+          if (h.d.model == model && h.d.order % 2 == up)
+            tiles(ts, mk_task(i, 0, 0, 0), NH, h.d.m - NH, NH, h.d.n - NH);
         }
         if (ts.empty()) continue;
         Launch& L = add(L_RHS, ts);
         L.stage = stage;
         L.outk = stage;
-        L.flags = model + 1;
+        L.flags = (model + 1) | (up ? 4 : 0);
       }
       // Euler inverts except at stage kforcing (unless diffusion);
       // Boussinesq inverts at every stage (core/euler.py:156-169,
@@ -3999,11 +4022,18 @@ static int run_prog_t(Batch& b, const std::vector<Launch>& prog, ProfSel* prof =
     const int nrep = timed ? PROF_REP : 1;
     for (int rep = 0; rep < nrep; rep++) switch (L.kind) {
       case L_RHS:
-        if (L.flags == 2)
-          F2D_LAUNCH((k_rhs<T, 2>), dim3(g), B2, 0, b.s, TK, b.dI, P, Q, b.B, b.dD, L.stage,
+        // flags: tracers, 4 upwind
+        if (L.flags == (2 | 4))
+          F2D_LAUNCH((k_rhs<T, 2, true>), dim3(g), B2, 0, b.s, TK, b.dI, P, Q, b.B, b.dD, L.stage,
+                     L.outk);
+        else if (L.flags == (1 | 4))
+          F2D_LAUNCH((k_rhs<T, 1, true>), dim3(g), B2, 0, b.s, TK, b.dI, P, Q, b.B, b.dD, L.stage,
+                     L.outk);
+        else if (L.flags == 2)
+          F2D_LAUNCH((k_rhs<T, 2, false>), dim3(g), B2, 0, b.s, TK, b.dI, P, Q, b.B, b.dD, L.stage,
                      L.outk);
         else
-          F2D_LAUNCH((k_rhs<T, 1>), dim3(g), B2, 0, b.s, TK, b.dI, P, Q, b.B, b.dD, L.stage,
+          F2D_LAUNCH((k_rhs<T, 1, false>), dim3(g), B2, 0, b.s, TK, b.dI, P, Q, b.B, b.dD, L.stage,
                      L.outk);
         break;
       case L_C2C:
