@@ -229,9 +229,10 @@ def cpu_model():
 
 def finest_tile_height(nx, ny, min_tiles):
     """Tile height of the finest-level smoother launches: the tallest of
-    16, 8, 4 rows (64 columns) giving at least min_tiles tiles."""
+    16, 8, 4 rows (64 columns) giving at least min_tiles tiles (0: the
+    library's default, 1024)."""
     if min_tiles <= 0:
-        return 16
+        min_tiles = 1024
     for ty in (16, 8):
         if nx * ny / (64.0 * ty) >= min_tiles:
             return ty

@@ -7,7 +7,7 @@ Two knobs shape the launches of a batch (``f2d_batch_tuning``):
   more levels there means fewer, but serial, phases per V-cycle.
 * ``min_tiles``: the fine phases use 64 x 16, 64 x 8 or 64 x 4 tiles, the
   tallest that still gives this many workgroups, so that small levels
-  spread over more compute units.
+  spread over more compute units (0: the default, 1024; 1: always 16 rows).
 * ``coarse_wave_cells``: inside the coarse kernel, levels up to this size
   run on a single wavefront (no workgroup barriers) instead of the whole
   workgroup.
@@ -36,7 +36,7 @@ from .grid import Grid
 from .param import Param
 
 BUDGETS = (0, 98304, 49152, 24576)
-MIN_TILES = (0, 1024, 4096, 1 << 24)
+MIN_TILES = (0, 1, 4096, 1 << 24)
 WAVE_CELLS = (256, 0)
 PERSIST = ()
 
@@ -57,7 +57,7 @@ def signature(pg, precision):
     for p, g in pg:
         k = "%s:%dx%d:%s" % (p.modelname, g.nx, g.ny, "perio" if g.geometry == "perio" else "wall")
         keys[k] = keys.get(k, 0) + 1
-    return "v2|" + precision + "|" + ",".join("%s*%d" % (k, keys[k]) for k in sorted(keys))
+    return "v3|" + precision + "|" + ",".join("%s*%d" % (k, keys[k]) for k in sorted(keys))
 
 
 def _cache_path():

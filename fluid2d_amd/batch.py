@@ -85,8 +85,8 @@ def _call(name, *args):
 
 class Tuning(C.Structure):
     """f2d_batch_tuning: coarse-kernel LDS budget (bytes, 0 = device
-    maximum), the minimum workgroup count of a fine phase (0 = always
-    16-row tiles), the largest coarse level (cells) run on one wavefront
+    maximum), the minimum workgroup count of a fine phase (0 = default 1024,
+    1 = always 16-row tiles), the largest coarse level (cells) run on one wavefront
     (-1 = default 256) and the persistent multigrid launches (workgroups per
     compute unit, 0 = one launch per phase)."""
     _fields_ = [("coarse_lds_budget", C.c_int), ("min_tiles", C.c_int),

@@ -3056,6 +3056,12 @@ constexpr double RR_STAGE_TILES_B = 512.;
 // the 128^2 and 64^2 levels at 1024^2) take tiles of 2 fine rows, twice the
 // workgroups, each with half the cells (-0.6 % per 1024^2 step)
 constexpr double RR_SMALL_TILES = 64.;
+// Default of a fine phase's least workgroup count (four per CU).  Tall tiles
+// on a small phase leave the chip idle: 8 x 256^2 FP64, per 4 steps, 4765 us
+// with 16 rows everywhere, 4060 at 256, 3956 at 1024, 4012 with 4 rows
+// everywhere; 32 mixed instances of 64^2..512^2, per 2 steps, 5115, 4998,
+// 4860, 5129; one 1024^2, per 4 steps, 7909, 6802, 6650, 6843.
+constexpr int MIN_TILES = 1024;
 // two-level restrictions of b: launches of at most RB2_TILES tiles of 8
 // output rows take tiles of RB2_TY_SMALL rows
 constexpr int RB2_TILES = 256, RB2_TY_SMALL = 4;
@@ -3140,12 +3146,18 @@ struct Builder {
 
   // Fine-phase tile height: the tallest of 16, 8, 4 rows that still gives
   // at least min_tiles workgroups over the cells of the phase (all
-  // instances at bottom-aligned level dd); min_tiles <= 0: always 16.
+  // instances at bottom-aligned level dd); min_tiles <= 0: MIN_TILES.
   int pick_ty_cells(double cells) const {
-    if (b.min_tiles <= 0) return TY;
+    const int least = b.min_tiles > 0 ? b.min_tiles : MIN_TILES;
     for (int ty = TY; ty > 4; ty /= 2)
-      if (cells / ((double)TX * ty) >= (double)b.min_tiles) return ty;
+      if (cells / ((double)TX * ty) >= (double)least) return ty;
     return 4;
+  }
+  // tile rows of a finest-level phase over the instances `who`
+  int pick_ty0(const std::vector<int>& who) const {
+    double cells = 0.;
+    for (int i : who) cells += (double)h_cells(i);
+    return pick_ty_cells(cells);
   }
   // tile rows of a fused down-leg phase: 2 on the smallest phases, else ty,
   // or the lowest of 8 and `most` (rows) that brings the phase to at most
@@ -3519,16 +3531,19 @@ struct Builder {
   // tendency, so their differences do not cancel in FP32.
   void invert_fast_refined(const std::vector<int>& who, int k) {
     std::vector<Task> rs;
+    const int ty = pick_ty0(who);
     for (int i : who) {
       HostInst& h = b.H[i];
       h.buf[0][0] = h.d.x0[0];
       h.buf[0][1] = h.d.x0[1];
       h.cur[0] = 0;
-      rr_tasks(i, 0, h.d.kp[k], h.d.k[k], h.d.L[0].b, rs);
+      rr_tasks(i, 0, h.d.kp[k], h.d.k[k], h.d.L[0].b, rs, ty / 2);
     }
     // FP64 defect b - A x0 with b = celltocorner(omega tendency) formed on
     // the fly, stored (T) as the level-0 rhs and restricted
-    add(L_RR, rs).flags = 1 | 32 | 64;
+    Launch& Lr = add(L_RR, rs);
+    Lr.flags = 1 | 32 | 64;
+    Lr.ty = ty;
     std::vector<int> st(b.ninst, 0);
     vcycle(who, st, 1, 0, false);
     vcycle(who, st, 0, 0, true);
@@ -3627,10 +3642,10 @@ struct Builder {
     vcycle(who, st, 0, 0, false);
     prog = &b.prog_init;
     std::vector<Task> rs;
-    rr_tasks(0, 0, 0, -1, -1, rs, pick_ty_cells((double)h_cells(0)) / 2);
+    rr_tasks(0, 0, 0, -1, -1, rs, pick_ty0(who) / 2);
     Launch& L = add(L_RR, rs);
     L.flags = 2;
-    L.ty = pick_ty_cells((double)h_cells(0));
+    L.ty = pick_ty0(who);
     fcycle_down(who, 0);
     coarse(who, 1, 0);
     fcycle_up(who, 0);
@@ -3655,11 +3670,12 @@ struct Builder {
       std::vector<Task> rs;
       for (int i : who) {
         HostInst& h = b.H[i];
-        rr_tasks(i, 0, psi(h), rhs(h), h.d.L[0].b, rs);
+        rr_tasks(i, 0, psi(h), rhs(h), h.d.L[0].b, rs, pick_ty0(who) / 2);
       }
       const int sp = spans_of(rs);
       Launch& L = add(L_RR, rs);
       L.flags = 1 | 4 | 8 | 32 | rhs_flag | (psi_q ? 128 : 0);  // FP64 outer residual
+      L.ty = pick_ty0(who);
       L.pred = pred;
       fold(what, sp, pred, maxite, tol);
     };
@@ -3838,9 +3854,12 @@ struct Builder {
         h.buf[0][0] = h.d.x0[0];
         h.buf[0][1] = h.d.x0[1];
         h.cur[0] = 0;
-        rr_tasks(i, 0, h.d.state + (long long)h.d.m * h.d.n, h.d.work, h.d.L[0].b, rs);
+        rr_tasks(i, 0, h.d.state + (long long)h.d.m * h.d.n, h.d.work, h.d.L[0].b, rs,
+                 pick_ty0(who) / 2);
       }
-      add(L_RR, rs).flags = 1 | 16 | 32;  // FP64 defect, stored (T) and restricted
+      Launch& Lr = add(L_RR, rs);
+      Lr.flags = 1 | 16 | 32;  // FP64 defect, stored (T) and restricted
+      Lr.ty = pick_ty0(who);
       vcycle(who, st, 1, 0, false);
       vcycle(who, st, 0, 0, false);
       std::vector<Task> up, fin;
@@ -4808,9 +4827,7 @@ static int hierarchy_build(Hierarchy& H, int nlev, const HierLevel* L, const uin
   memset(&dyn, 0, sizeof dyn);
   dyn.run = dyn.active = 1;
   ECHK(hipMemcpy(b.dD, &dyn, sizeof dyn, hipMemcpyHostToDevice));
-  // the launch shapes the autotuner picks for one grid
-  const f2d_batch_tuning t{0, 1024, 0, 0};
-  ETRY(apply_tuning(b, &t));
+  ETRY(apply_tuning(b, nullptr));
   ECHK(hipStreamCreateWithFlags(&b.s, hipStreamNonBlocking));
   return F2D_OK;
 }

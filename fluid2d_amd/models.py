@@ -298,7 +298,7 @@ class EngineModel:
         # model on a scratch batch, then cached)
         from . import autotune
         cands = [{"coarse_lds_budget": 0, "min_tiles": mt, "coarse_wave_cells": wc}
-                 for mt in (0, 1024, 4096) for wc in (256, 0)]
+                 for mt in (0, 512, 4096) for wc in (256, 0)]
         tuning = None
         if getattr(param, "autotune", True):
             tuning, _ = autotune.tune([(param, grid)], "fp64", cands=cands)

@@ -279,8 +279,8 @@ const char *f2d_batch_last_error(void);
  *   kernel (0 = the device maximum); levels are handed to it from the
  *   coarsest up while they fit.
  * min_tiles: a fine-level phase uses the tallest tile (16, 8 or 4 rows of
- *   64 cells) that still gives at least this many workgroups (0 = always
- *   16 rows).
+ *   64 cells) that still gives at least this many workgroups (0 = the
+ *   default, 1024; 1 = always 16 rows).
  * coarse_wave_cells: inside the coarse kernel, levels of at most this many
  *   cells (halo included) run on one wavefront without workgroup barriers;
  *   larger ones use the whole workgroup (0 = none on one wavefront;
