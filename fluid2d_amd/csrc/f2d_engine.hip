@@ -1161,6 +1161,34 @@ __global__ void __launch_bounds__(NTH) k_restrict_b2(const Task* __restrict__ ta
   }
 }
 
+// A cell's operator row in registers: the eight couplings offdiag_2d reads
+// and the centre A_5 (residual_2d); the arguments are literals after
+// inlining
+template <typename T>
+struct ARow {
+  T a0, a1, a2, a3, a4, a3e, a2s, a1s, a0s;
+  __device__ __forceinline__ T operator()(int k, int dj, int di) const {
+    if (dj == 0 && di == 0)
+      return k == 0 ? a0 : (k == 1 ? a1 : (k == 2 ? a2 : (k == 3 ? a3 : a4)));
+    return k == 3 ? a3e : (k == 2 ? a2s : (k == 1 ? a1s : a0s));
+  }
+};
+// the row of the cell at element e of a level's five planes (PL values each,
+// row length n), every load at once
+template <typename T>
+__device__ __forceinline__ void load_row(ARow<T>& r, const T* A, uint32_t PL, uint32_t n,
+                                         uint32_t e) {
+  r.a4 = ld32(A, 4 * PL + e);
+  r.a0 = ld32(A, e);
+  r.a1 = ld32(A, PL + e);
+  r.a2 = ld32(A, 2 * PL + e);
+  r.a3 = ld32(A, 3 * PL + e);
+  r.a3e = ld32(A, 3 * PL + e + 1);
+  r.a2s = ld32(A, 2 * PL + e + n - 1);
+  r.a1s = ld32(A, PL + e + n);
+  r.a0s = ld32(A, e + n + 1);
+}
+
 // ---------------------------------------------------------------------------
 // k_smooth_rr: the down-leg of a V-cycle on a level below the finest entered
 // with x = 0 (hierarchy.py:103-108 for lev > lev1: smooth, residual,
@@ -1208,6 +1236,21 @@ __device__ __forceinline__ int wrap_img(int g, int m) {
   while (g < NH) g += M;
   while (g >= m - NH) g -= M;
   return g;
+}
+// Image of position g, at most one period away when `one` (uniform over the
+// workgroup): two selects; else any number of periods (levels narrower than
+// the tile's region).
+__device__ __forceinline__ int wrap_pos(int g, int m, bool one) {
+  const int M = m - 2 * NH;
+  int r = g < NH ? g + M : g;
+  r = r >= m - NH ? r - M : r;
+  if (!one) r = wrap_img(g, m);
+  return r;
+}
+// whether positions lo .. hi of an axis of m need at most one period
+__device__ __forceinline__ bool one_period(int lo, int hi, int m) {
+  const int M = m - 2 * NH;
+  return lo >= NH - M && hi < m - NH + M;
 }
 
 // X0: 1 the level is entered with x = 0 (a V-cycle's descent), 3 with
@@ -1478,6 +1521,12 @@ __global__ void __launch_bounds__(NTH) k_smooth_rr(const Task* __restrict__ task
 // its images), so the values equal the launch-per-level ones bit for bit.
 // Tile origins are odd (NH plus multiples of the even tile sizes): fine
 // region row rr lies over coarse region row (rr + 1) / 2, and so on down.
+//
+// A chain of six phases; what bounds it is their latency.  The thread that
+// owns a cell in a level's first sweep owns it in the second, its operator
+// row and c1 / |A_5| in registers, loaded with everything else: one memory
+// round trip instead of one more per sweep.  Whole steps: 1024^2 1647 -> 1610
+// us, 2048 x 1024 Boussinesq 1147 -> 1133, 384 x 192 mixed 392 -> 384.
 // ---------------------------------------------------------------------------
 // NTH: threads per workgroup, (64, NTH / 64); its launches are small (at
 // most 256 tiles), so 1024 threads make each phase one pass over its region.
@@ -1494,21 +1543,18 @@ __global__ void __launch_bounds__(NTH) k_up2(const Task* __restrict__ tasks,
   constexpr int C2H = CH + 4, C2W = CW + 4;          // coarse x0
   constexpr int DH = C2H / 2 + 2, DW = C2W / 2 + 2;  // next coarser x under the coarse x0
   constexpr int ND = DH * DW, NC2 = C2H * C2W, NC1 = C1H * C1W, NX = XH * XW, NJ = JH * JW;
-  constexpr int ITD = (ND + NT - 1) / NT, ITC2 = (NC2 + NT - 1) / NT, ITC1 = (NC1 + NT - 1) / NT;
+  constexpr int ITD = (ND + NT - 1) / NT, ITC2 = (NC2 + NT - 1) / NT;
   constexpr int ITX = (NX + NT - 1) / NT, ITJ = (NJ + NT - 1) / NT;
   __shared__ T xd[DH][DW];
   __shared__ int8_t md[DH][DW];
   __shared__ T x0c[C2H][C2W];
   __shared__ int8_t mc[C2H][C2W];
-  __shared__ T bc[C1H][C1W];
-  __shared__ uint32_t ic[C1H][C1W];  // image cell index (coarse level)
   __shared__ T j1c[C1H][C1W];
   __shared__ T cx[CH][CW];
   __shared__ T xs[XH][XW];
   __shared__ int8_t mf[XH][XW];
-  __shared__ T bs[JH][JW];
-  __shared__ uint32_t jf[JH][JW];  // image cell index (fine level)
   __shared__ T j1[JH][JW];
+  static_assert(NC1 <= NT, "one coarse first-sweep cell per thread");
   const int ti = task_index();
   const Task tk = tasks[ti];
   const InstD& in = I[tk.inst];
@@ -1520,42 +1566,46 @@ __global__ void __launch_bounds__(NTH) k_up2(const Task* __restrict__ tasks,
   const int8_t* mskf = B + tk.msk;
   const int8_t* mskc = B + tk.msk2;
   const int8_t* mskd = B + tk.msk3;
+  const bool one = one_period(y0 - 2, y0 + XH, m) && one_period(x0 - 2, x0 + XW, n) &&
+                   one_period(cy0 - 2, cy0 + C2H, m2) && one_period(cx0 - 2, cx0 + C2W, n2) &&
+                   one_period(dy0, dy0 + DH, m3) && one_period(dx0, dx0 + DW, n3);
   // every load of the tile issued before the first is used
-  T vd[ITD], vc2[ITC2], vb1[ITC1], vx[ITX], vj[ITJ];
+  T vd[ITD], vc2[ITC2], vb1, vx[ITX], vj[ITJ];
   int8_t wd[ITD], wc2[ITC2], wx[ITX];
-  uint32_t uc1[ITC1], uj[ITJ];
+  ARow<T> rc, rf[ITJ];
 #pragma unroll
   for (int it = 0; it < ITD; it++) {
     const int q = min(tid + it * NT, ND - 1), a = q / DW, c = q - a * DW;
-    const uint32_t e = at32(wrap_img(dy0 + a, m3), wrap_img(dx0 + c, n3), n3);
+    const uint32_t e = at32(wrap_pos(dy0 + a, m3, one), wrap_pos(dx0 + c, n3, one), n3);
     vd[it] = ld32(Q + tk.xcc, e);
     wd[it] = ld32(mskd, e);
   }
 #pragma unroll
   for (int it = 0; it < ITC2; it++) {
     const int q = min(tid + it * NT, NC2 - 1), a = q / C2W, c = q - a * C2W;
-    const uint32_t e = at32(wrap_img(cy0 - 2 + a, m2), wrap_img(cx0 - 2 + c, n2), n2);
+    const uint32_t e = at32(wrap_pos(cy0 - 2 + a, m2, one), wrap_pos(cx0 - 2 + c, n2, one), n2);
     vc2[it] = ld32(Q + tk.xin2, e);
     wc2[it] = ld32(mskc, e);
   }
-#pragma unroll
-  for (int it = 0; it < ITC1; it++) {
-    const int q = min(tid + it * NT, NC1 - 1), a = q / C1W, c = q - a * C1W;
-    uc1[it] = at32(wrap_img(cy0 - 1 + a, m2), wrap_img(cx0 - 1 + c, n2), n2);
-    vb1[it] = ld32(Q + tk.b2, uc1[it]);
+  const int ca = min(tid, NC1 - 1) / C1W, cc = min(tid, NC1 - 1) - ca * C1W;
+  {
+    const uint32_t e = at32(wrap_pos(cy0 - 1 + ca, m2, one), wrap_pos(cx0 - 1 + cc, n2, one), n2);
+    vb1 = ld32(Q + tk.b2, e);
+    load_row(rc, Q + tk.A2, (uint32_t)m2 * (uint32_t)n2, (uint32_t)n2, e);
   }
 #pragma unroll
   for (int it = 0; it < ITX; it++) {
     const int q = min(tid + it * NT, NX - 1), a = q / XW, c = q - a * XW;
-    const uint32_t e = at32(wrap_img(y0 - 2 + a, m), wrap_img(x0 - 2 + c, n), n);
+    const uint32_t e = at32(wrap_pos(y0 - 2 + a, m, one), wrap_pos(x0 - 2 + c, n, one), n);
     vx[it] = ld32(Q + tk.xin, e);
     wx[it] = ld32(mskf, e);
   }
 #pragma unroll
   for (int it = 0; it < ITJ; it++) {
     const int q = min(tid + it * NT, NJ - 1), a = q / JW, c = q - a * JW;
-    uj[it] = at32(wrap_img(y0 - 1 + a, m), wrap_img(x0 - 1 + c, n), n);
-    vj[it] = ld32(Q + tk.b, uj[it]);
+    const uint32_t e = at32(wrap_pos(y0 - 1 + a, m, one), wrap_pos(x0 - 1 + c, n, one), n);
+    vj[it] = ld32(Q + tk.b, e);
+    load_row(rf[it], Q + tk.A, (uint32_t)m * (uint32_t)n, (uint32_t)n, e);
   }
   if (skip(dyn, tk.inst, pred)) return;
 #pragma unroll
@@ -1572,25 +1622,9 @@ __global__ void __launch_bounds__(NTH) k_up2(const Task* __restrict__ tasks,
     if (q < NC2) mc[a][c] = wc2[it];
   }
 #pragma unroll
-  for (int it = 0; it < ITC1; it++) {
-    const int q = tid + it * NT, a = q / C1W, c = q - a * C1W;
-    if (q < NC1) {
-      bc[a][c] = vb1[it];
-      ic[a][c] = uc1[it];
-    }
-  }
-#pragma unroll
   for (int it = 0; it < ITX; it++) {
     const int q = tid + it * NT, a = q / XW, c = q - a * XW;
     if (q < NX) mf[a][c] = wx[it];
-  }
-#pragma unroll
-  for (int it = 0; it < ITJ; it++) {
-    const int q = tid + it * NT, a = q / JW, c = q - a * JW;
-    if (q < NJ) {
-      bs[a][c] = vj[it];
-      jf[a][c] = uj[it];
-    }
   }
   __syncthreads();
   // prolongation at region position (rr, cc) from the coarser tile X with
@@ -1618,31 +1652,25 @@ __global__ void __launch_bounds__(NTH) k_up2(const Task* __restrict__ tasks,
   }
   __syncthreads();
   const T c1 = T(in.omega), c2 = T(1. - in.omega);
-  const T* Ac = Q + tk.A2;
-  const T* Af = Q + tk.A;
-  const size_t PLc = (size_t)m2 * n2, PLf = (size_t)m * n;
-  auto Aat = [&](const T* A, size_t PL, int nn, uint32_t e) {
-    const APlanes<T> Ap{A, PL, e};
-    return [=](int k, int dj, int di) { return Ap(k, (ptrdiff_t)dj * nn + di); };
-  };
+  const T c3c = c1 / fabs(rc.a4);
   // coarse first sweep (region less one ring of x0), second sweep on the
   // prolongation's region; the cells the tile lies over are stored
-  for (int q = tid; q < NC1; q += NT) {
-    const int a = q / C1W, c = q - a * C1W;
-    j1c[a][c] = jacobi_2d<T>(mc[a + 1][c + 1], bc[a][c], c1, c2, Aat(Ac, PLc, n2, ic[a][c]),
-                             [&](int dj, int di) { return x0c[a + 1 + dj][c + 1 + di]; });
+  const int8_t mkc = mc[ca + 1][cc + 1];
+  if (tid < NC1) {
+    const T v = jacobi_c3_2d<T>(vb1, c3c, c2, rc,
+                                [&](int dj, int di) { return x0c[ca + 1 + dj][cc + 1 + di]; });
+    j1c[ca][cc] = mkc == 0 ? T(0) : v;
   }
   __syncthreads();
-  T* xoc = Q + tk.xc;
-  for (int q = tid; q < CH * CW; q += NT) {
-    const int a = q / CW, c = q - a * CW;
-    const T v = jacobi_2d<T>(mc[a + 2][c + 2], bc[a + 1][c + 1], c1, c2,
-                             Aat(Ac, PLc, n2, ic[a + 1][c + 1]),
-                             [&](int dj, int di) { return j1c[a + 1 + dj][c + 1 + di]; });
+  if (tid < NC1 && ca >= 1 && ca < C1H - 1 && cc >= 1 && cc < C1W - 1) {
+    const int a = ca - 1, c = cc - 1;
+    T v = jacobi_c3_2d<T>(vb1, c3c, c2, rc,
+                          [&](int dj, int di) { return j1c[ca + dj][cc + di]; });
+    if (mkc == 0) v = T(0);
     cx[a][c] = v;
     const int J = cy0 + a, Ic = cx0 + c;
     if (a >= 2 && a < 2 + TYV / 2 && c >= 2 && c < 2 + TX2 && J < m2 - NH && Ic < n2 - NH)
-      store_img_mask32<T>(xoc, nullptr, J, Ic, v, m2, n2);
+      store_img_mask32<T>(Q + tk.xc, nullptr, J, Ic, v, m2, n2);
   }
   __syncthreads();
   // fine x0 = x + I(coarse x)
@@ -1652,21 +1680,28 @@ __global__ void __launch_bounds__(NTH) k_up2(const Task* __restrict__ tasks,
     if (q < NX) xs[a][c] = vx[it] + ip(cx, mc, 2, mf[a][c], a, c);  // cx = mc's region + 2
   }
   __syncthreads();
-  for (int q = tid; q < NJ; q += NT) {
-    const int a = q / JW, c = q - a * JW;
-    j1[a][c] = jacobi_2d<T>(mf[a + 1][c + 1], bs[a][c], c1, c2, Aat(Af, PLf, n, jf[a][c]),
-                            [&](int dj, int di) { return xs[a + 1 + dj][c + 1 + di]; });
+  T c3f[ITJ];
+#pragma unroll
+  for (int it = 0; it < ITJ; it++) {
+    const int q = tid + it * NT, a = q / JW, c = q - a * JW;
+    if (q < NJ) {
+      c3f[it] = c1 / fabs(rf[it].a4);
+      const T v = jacobi_c3_2d<T>(vj[it], c3f[it], c2, rf[it],
+                                  [&](int dj, int di) { return xs[a + 1 + dj][c + 1 + di]; });
+      j1[a][c] = mf[a + 1][c + 1] == 0 ? T(0) : v;
+    }
   }
   __syncthreads();
   T* xo = Q + tk.xout;
-  for (int q = tid; q < TYV * TX; q += NT) {
-    const int a = q / TX, c = q - a * TX;
-    const int J = y0 + a, Ic = x0 + c;
-    if (J >= m - NH || Ic >= n - NH) continue;
-    const T v = jacobi_2d<T>(mf[a + 2][c + 2], bs[a + 1][c + 1], c1, c2,
-                             Aat(Af, PLf, n, jf[a + 1][c + 1]),
-                             [&](int dj, int di) { return j1[a + 1 + dj][c + 1 + di]; });
-    store_img_mask32<T>(xo, nullptr, J, Ic, v, m, n);
+#pragma unroll
+  for (int it = 0; it < ITJ; it++) {
+    const int q = tid + it * NT, a = q / JW, c = q - a * JW;
+    const int J = y0 + a - 1, Ic = x0 + c - 1;
+    if (q >= NJ || a < 1 || a >= JH - 1 || c < 1 || c >= JW - 1 || J >= m - NH || Ic >= n - NH)
+      continue;
+    const T v = jacobi_c3_2d<T>(vj[it], c3f[it], c2, rf[it],
+                                [&](int dj, int di) { return j1[a + dj][c + di]; });
+    store_img_mask32<T>(xo, nullptr, J, Ic, mf[a + 1][c + 1] == 0 ? T(0) : v, m, n);
   }
 }
 
@@ -1902,19 +1937,6 @@ __device__ __forceinline__ void c_interp(const CL<T, TA>& F, const CL<T, TA>& C,
     }
   sy.end(cnt);
 }
-
-// A cell's operator row in registers: the eight couplings offdiag_2d reads
-// and the centre A_5 (residual_2d); the arguments are literals after
-// inlining
-template <typename T>
-struct ARow {
-  T a0, a1, a2, a3, a4, a3e, a2s, a1s, a0s;
-  __device__ __forceinline__ T operator()(int k, int dj, int di) const {
-    if (dj == 0 && di == 0)
-      return k == 0 ? a0 : (k == 1 ? a1 : (k == 2 ? a2 : (k == 3 ? a3 : a4)));
-    return k == 3 ? a3e : (k == 2 ? a2s : (k == 1 ? a1s : a0s));
-  }
-};
 
 // An interior cell held by its owning thread: position, operator row,
 // c1 / |A_5|, rhs and mask (read once per level visit)
