@@ -1257,15 +1257,20 @@ __device__ __forceinline__ bool one_period(int lo, int hi, int m) {
 // x = I(x of the coarser level) (an F-cycle's V-cycle from this level,
 // hierarchy.py:145-151); the prolongation is evaluated at the images too (the
 // coarse x and both masks are stored with their images).
-// STAGE: the five operator planes on the region (plus the row and the
-// columns the stencil reaches past it) are loaded with the tile, at their
-// images, and the sweeps and residuals read them from LDS: one memory round
-// trip for the launch instead of one per phase (the small launches of the
-// mid levels, whose time is those round trips).  NTH: threads per
-// workgroup, (64, NTH / 64); 1024 for launches of at most two workgroups
-// per CU, where each phase is then one pass over its region instead of
-// several.
-template <typename T, int TY2V, int X0, int STAGE = 0, int NTH = 256>
+//
+// What bounds it: the latency of its phases (a load, two sweeps, the
+// residual, the restriction).  The thread that owns a region cell owns it in
+// every phase, with its operator row, c1 / |A_5|, rhs and mask in registers:
+// one memory round trip, and each phase reads only its neighbours' x from
+// LDS.  The first sweep from x = 0 is 0 + c3 (0 - b): every product with x is
+// a zero, and a zero sum's sign is lost in the final sum with +0.  With the
+// operator read by each phase (from LDS copies on small launches) the 512^2
+// level took 8.4 us, 64^2 5.0, 1024 x 512 15.8; so 6.4, 4.3, 10.1 (of which
+// about 2 are the launch).  Whole steps: 1024^2 1610 -> 1529 us, 2048 x 1024
+// Boussinesq 1133 -> 1073.
+// NTH: threads of a workgroup, (64, NTH / 64).
+constexpr int rr_threads(int ty2) { return ty2 == 1 ? 512 : (ty2 == 2 ? 640 : (ty2 == 4 ? 960 : 768)); }
+template <typename T, int TY2V, int X0, int NTH = rr_threads(TY2V)>
 __global__ void __launch_bounds__(NTH) k_smooth_rr(const Task* __restrict__ tasks,
                                                    const InstD* __restrict__ I, T* Q,
                                                    const int8_t* __restrict__ B,
@@ -1276,17 +1281,11 @@ __global__ void __launch_bounds__(NTH) k_smooth_rr(const Task* __restrict__ task
   constexpr int H1 = RY + 2, W1 = RX + 2;             // second sweep
   constexpr int H2 = RY + 4, W2 = RX + 4;             // first sweep, rhs, mask
   constexpr int H3 = X0 == 3 ? RY + 6 : 1, W3 = X0 == 3 ? RX + 6 : 1;  // x0 (prolongation)
-  constexpr int NR2 = H2 * W2, IT2 = (NR2 + NT - 1) / NT;
+  constexpr int NR2 = H2 * W2, IT = (NR2 + NT - 1) / NT;
   __shared__ T x0s[H3][W3];
   __shared__ T x1s[H2][W2];
-  __shared__ T bs2[H2][W2];
   __shared__ T x2s[H1][W1];
   __shared__ T rs[RY][RX];
-  __shared__ int8_t ms[H2][W2];
-  __shared__ uint32_t cs[STAGE ? 1 : H2][STAGE ? 1 : W2];  // image cell index of each region position
-  // staged operator: rows [gy, gy + H2], columns [gx - 1, gx + W2]
-  constexpr int HA = H2 + 1, WA = W2 + 2, NA = HA * WA, ITA = STAGE ? (NA + NT - 1) / NT : 1;
-  __shared__ T As[STAGE ? 5 : 1][STAGE ? HA : 1][STAGE ? WA : 1];
   const int ti = task_index();
 #ifdef F2D_PHASE_STAMPS
   const unsigned long long st0 = wall_clock64();
@@ -1301,37 +1300,33 @@ __global__ void __launch_bounds__(NTH) k_smooth_rr(const Task* __restrict__ task
 #endif
   const InstD& in = I[tk.inst];
   const int m1 = tk.m, n1 = tk.n, m2 = tk.m2, n2 = tk.n2;
-  const size_t PL = (size_t)m1 * n1;
+  const uint32_t PL = (uint32_t)m1 * (uint32_t)n1;
   const int8_t* msk = B + tk.msk;
   const int8_t* msk2 = B + tk.msk2;
-  const T* A = Q + tk.A;
-  const T* b = Q + tk.b;
   const int tid = threadIdx.y * 64 + threadIdx.x;
   const int fy0 = 2 * tk.y0 - 3, fx0 = 2 * tk.x0 - 3;  // first residual point
   const int gy = fy0 - 2, gx = fx0 - 2;                // first-sweep region origin
-  // rhs and mask of the first sweep's region, every load issued before use
-  T bv[IT2];
-  int8_t mv[IT2];
-  uint32_t cv[IT2];
+  const bool one = one_period(gy - 1, gy + H2, m1) && one_period(gx - 1, gx + W2, n1);
+  // rhs, mask and operator row of the owned cells, at their images, every
+  // load issued before use
+  T bv[IT];
+  int8_t mv[IT];
+  ARow<T> row[IT];
 #pragma unroll
-  for (int it = 0; it < IT2; it++) {
+  for (int it = 0; it < IT; it++) {
     const int q = min(tid + it * NT, NR2 - 1);
     const int rr = q / W2, cc = q - rr * W2;
-    cv[it] = at32(wrap_img(gy + rr, m1), wrap_img(gx + cc, n1), n1);
-    bv[it] = ld32(b, cv[it]);
-    mv[it] = ld32(msk, cv[it]);
+    const uint32_t e = at32(wrap_pos(gy + rr, m1, one), wrap_pos(gx + cc, n1, one), n1);
+    bv[it] = ld32(Q + tk.b, e);
+    mv[it] = ld32(msk, e);
+    load_row(row[it], Q + tk.A, PL, (uint32_t)n1, e);
   }
-  T av[5][ITA];
-  if constexpr (STAGE != 0) {
-#pragma unroll
-    for (int it = 0; it < ITA; it++) {
-      const int q = min(tid + it * NT, NA - 1);
-      const int rr = q / WA, cc = q - rr * WA;
-      const uint32_t e = at32(wrap_img(gy + rr, m1), wrap_img(gx - 1 + cc, n1), n1);
-#pragma unroll
-      for (int k = 0; k < 5; k++) av[k][it] = ld32(A, (uint32_t)k * (uint32_t)PL + e);
-    }
-  }
+  // the coarse mask of the points restricted
+  constexpr int NC = TY2V * TX2;
+  static_assert(NC <= NT, "one coarse cell per thread");
+  const int ry = tid / TX2, rx = tid - ry * TX2, J2 = tk.y0 + ry, I2 = tk.x0 + rx;
+  const bool co = tid < NC && J2 < m2 - NH && I2 < n2 - NH;
+  const int8_t mc = ld32(msk2, co ? at32(J2, I2, n2) : 0u);
   // X0 3: x = I(xc) on the first sweep's region plus one ring.  Fine row
   // gy - 1 + rr (gy odd) lies over coarse row cy + rr / 2, so the coarse x
   // and mask under the region and the fine mask on it are loaded at their
@@ -1342,17 +1337,17 @@ __global__ void __launch_bounds__(NTH) k_smooth_rr(const Task* __restrict__ task
   constexpr int ITC3 = X0 == 3 ? (NC3 + NT - 1) / NT : 1, ITM3 = X0 == 3 ? (NM3 + NT - 1) / NT : 1;
   __shared__ T cx3[CH3][CW3];
   __shared__ int8_t cm3[CH3][CW3];
-  __shared__ int8_t m13[H3][W3];
   const int cy = (gy + 1) >> 1, cxo = (gx + 1) >> 1;
   T c3v[ITC3];
   int8_t s3v[ITC3], m3v[ITM3];
   if constexpr (X0 == 3) {
     const T* xc = Q + tk.xc;
+    const bool onec = one_period(cy, cy + CH3, m2) && one_period(cxo, cxo + CW3, n2);
 #pragma unroll
     for (int it = 0; it < ITC3; it++) {
       const int q = min(tid + it * NT, NC3 - 1);
       const int a = q / CW3, bb = q - a * CW3;
-      const uint32_t c = at32(wrap_img(cy + a, m2), wrap_img(cxo + bb, n2), n2);
+      const uint32_t c = at32(wrap_pos(cy + a, m2, onec), wrap_pos(cxo + bb, n2, onec), n2);
       c3v[it] = ld32(xc, c);
       s3v[it] = ld32(msk2, c);
     }
@@ -1360,33 +1355,11 @@ __global__ void __launch_bounds__(NTH) k_smooth_rr(const Task* __restrict__ task
     for (int it = 0; it < ITM3; it++) {
       const int q = min(tid + it * NT, NM3 - 1);
       const int rr = q / W3, cc = q - rr * W3;
-      m3v[it] = ld32(msk, at32(wrap_img(gy - 1 + rr, m1), wrap_img(gx - 1 + cc, n1), n1));
+      m3v[it] = ld32(msk, at32(wrap_pos(gy - 1 + rr, m1, one), wrap_pos(gx - 1 + cc, n1, one), n1));
     }
   }
   if (skip(dyn, tk.inst, pred)) return;
   F2D_RSTAMP(tk.lev, 2);
-#pragma unroll
-  for (int it = 0; it < IT2; it++) {
-    const int q = tid + it * NT;
-    if (q < NR2) {
-      const int rr = q / W2, cc = q - rr * W2;
-      bs2[rr][cc] = bv[it];
-      ms[rr][cc] = mv[it];
-      if constexpr (STAGE == 0) cs[rr][cc] = cv[it];
-    }
-  }
-  if constexpr (STAGE != 0) {
-#pragma unroll
-    for (int it = 0; it < ITA; it++) {
-      const int q = tid + it * NT;
-      if (q < NA) {
-        const int rr = q / WA, cc = q - rr * WA;
-#pragma unroll
-        for (int k = 0; k < 5; k++) As[k][rr][cc] = av[k][it];
-      }
-    }
-    if constexpr (X0 == 1) __syncthreads();  // (X0 3 synchronises below)
-  }
   if constexpr (X0 == 3) {
 #pragma unroll
     for (int it = 0; it < ITC3; it++) {
@@ -1397,16 +1370,11 @@ __global__ void __launch_bounds__(NTH) k_smooth_rr(const Task* __restrict__ task
         cm3[a][bb] = s3v[it];
       }
     }
+    __syncthreads();
 #pragma unroll
     for (int it = 0; it < ITM3; it++) {
       const int q = tid + it * NT;
-      if (q < NM3) {
-        const int rr = q / W3, cc = q - rr * W3;
-        m13[rr][cc] = m3v[it];
-      }
-    }
-    __syncthreads();
-    for (int q = tid; q < NM3; q += NT) {
+      if (q >= NM3) continue;
       const int rr = q / W3, cc = q - rr * W3;
       const int a = rr >> 1, bb = cc >> 1;
       IpOps<T> o;
@@ -1418,54 +1386,44 @@ __global__ void __launch_bounds__(NTH) k_smooth_rr(const Task* __restrict__ task
       o.sb = cm3[a][bb + 1];
       o.sc = cm3[a + 1][bb];
       o.sd = cm3[a + 1][bb + 1];
-      o.m1 = m13[rr][cc];
+      o.m1 = m3v[it];
       o.par = ((gx - 1 + cc) & 1) | (((gy - 1 + rr) & 1) << 1);
       x0s[rr][cc] = ip_eval<T>(o);
     }
     __syncthreads();
   }
   const T c1 = T(in.omega), c2 = T(1. - in.omega);
-  auto Aat = [&](uint32_t c) {
-    const APlanes<T> Ap{A, PL, c};
-    return [=](int k, int dj, int di) { return Ap(k, (ptrdiff_t)dj * n1 + di); };
-  };
-  // the operator of region position (rr, cc): from LDS when staged, else at
-  // the position's image in the level's planes
-  auto Aop = [&](int rr, int cc, uint32_t e) {
-    if constexpr (STAGE != 0) {
-      (void)e;
-      return [&, rr, cc](int k, int dj, int di) { return As[k][rr + dj][cc + 1 + di]; };
-    } else {
-      (void)rr;
-      (void)cc;
-      return Aat(e);
-    }
-  };
-  // first sweep on the whole region (rhs from registers), from x = 0 or
-  // from the prolongation
+  T c3[IT];
+  // first sweep on the whole region, from x = 0 or from the prolongation
 #pragma unroll
-  for (int it = 0; it < IT2; it++) {
+  for (int it = 0; it < IT; it++) {
     const int q = tid + it * NT;
+    c3[it] = c1 / fabs(row[it].a4);
     if (q < NR2) {
       const int rr = q / W2, cc = q - rr * W2;
+      T v;
       if constexpr (X0 == 3)
-        x1s[rr][cc] = jacobi_2d<T>(mv[it], bv[it], c1, c2, Aop(rr, cc, cv[it]),
-                                   [&](int dj, int di) { return x0s[rr + 1 + dj][cc + 1 + di]; });
+        v = jacobi_c3_2d<T>(bv[it], c3[it], c2, row[it],
+                            [&](int dj, int di) { return x0s[rr + 1 + dj][cc + 1 + di]; });
       else
-        x1s[rr][cc] = jacobi_2d<T>(mv[it], bv[it], c1, c2, Aop(rr, cc, cv[it]),
-                                   [](int, int) { return T(0); });
+        v = T(0) + c3[it] * (T(0) - bv[it]);
+      x1s[rr][cc] = mv[it] == 0 ? T(0) : v;
     }
   }
   __syncthreads();
   F2D_RSTAMP(tk.lev, 3);
   // second sweep on the region less one ring
-  constexpr int NR1 = H1 * W1;
-  for (int q = tid; q < NR1; q += NT) {
-    const int r1 = q / W1, c1i = q - r1 * W1;
-    const int rr = r1 + 1, cc = c1i + 1;
-    x2s[r1][c1i] = jacobi_2d<T>(ms[rr][cc], bs2[rr][cc], c1, c2,
-                                Aop(rr, cc, STAGE ? 0u : cs[STAGE ? 0 : rr][STAGE ? 0 : cc]),
-                                [&](int dj, int di) { return x1s[rr + dj][cc + di]; });
+  T x2[IT];
+#pragma unroll
+  for (int it = 0; it < IT; it++) {
+    const int q = tid + it * NT, rr = q / W2, cc = q - rr * W2;
+    x2[it] = T(0);
+    if (rr >= 1 && rr < H2 - 1 && cc >= 1 && cc < W2 - 1) {
+      const T v = jacobi_c3_2d<T>(bv[it], c3[it], c2, row[it],
+                                  [&](int dj, int di) { return x1s[rr + dj][cc + di]; });
+      x2[it] = mv[it] == 0 ? T(0) : v;
+      x2s[rr - 1][cc - 1] = x2[it];
+    }
   }
   __syncthreads();
   F2D_RSTAMP(tk.lev, 4);
@@ -1473,33 +1431,29 @@ __global__ void __launch_bounds__(NTH) k_smooth_rr(const Task* __restrict__ task
   // fine cells (local rows/cols [0, 2*T) off the halo, under the coarse
   // interior) stored with their images
   T* xout = Q + tk.xout;
-  constexpr int NRR = RY * RX;
-  for (int q = tid; q < NRR; q += NT) {
-    const int r0 = q / RX, c0 = q - r0 * RX;
-    const int rr = r0 + 2, cc = c0 + 2;
-    rs[r0][c0] = residual_2d<T>(ms[rr][cc], bs2[rr][cc],
-                                Aop(rr, cc, STAGE ? 0u : cs[STAGE ? 0 : rr][STAGE ? 0 : cc]),
-                                [&](int dj, int di) { return x2s[r0 + 1 + dj][c0 + 1 + di]; });
+#pragma unroll
+  for (int it = 0; it < IT; it++) {
+    const int q = tid + it * NT, rr = q / W2, cc = q - rr * W2;
+    const int r0 = rr - 2, c0 = cc - 2;
+    if (r0 < 0 || r0 >= RY || c0 < 0 || c0 >= RX) continue;
+    rs[r0][c0] = residual_2d<T>(mv[it], bv[it], row[it], [&](int dj, int di) {
+      return x2s[r0 + 1 + dj][c0 + 1 + di];
+    });
     const int jf = fy0 + r0, if_ = fx0 + c0;
     if (r0 < 2 * TY2V && c0 < 2 * TX2 && jf < m1 - NH && if_ < n1 - NH &&
         (tk.y0 + r0 / 2) < m2 - NH && (tk.x0 + c0 / 2) < n2 - NH)
-      store_img_mask32<T>(xout, nullptr, jf, if_, x2s[r0 + 1][c0 + 1], m1, n1);
+      store_img_mask32<T>(xout, nullptr, jf, if_, x2[it], m1, n1);
   }
   __syncthreads();
   F2D_RSTAMP(tk.lev, 5);
   // full weighting onto the coarse tile (+ images)
-  T* b2 = Q + in.L[tk.lev + 1].b;
-  constexpr int NC = TY2V * TX2;
-  for (int q = tid; q < NC; q += NT) {
-    const int ry = q / TX2, rx = q - ry * TX2;
-    const int J2 = tk.y0 + ry, I2 = tk.x0 + rx;
-    if (J2 >= m2 - NH || I2 >= n2 - NH) continue;
+  if (co) {
     T v = T(0);
-    if (ld32(msk2, at32(J2, I2, n2)) != 0) {
-      const int cy = 2 * ry + 1, cx = 2 * rx + 1;
-      v = restrict_r<T>([&](int dj, int di) { return rs[cy + dj][cx + di]; });
+    if (mc != 0) {
+      const int y = 2 * ry + 1, x = 2 * rx + 1;
+      v = restrict_r<T>([&](int dj, int di) { return rs[y + dj][x + di]; });
     }
-    store_img_mask32<T>(b2, nullptr, J2, I2, v, m2, n2);
+    store_img_mask32<T>(Q + in.L[tk.lev + 1].b, nullptr, J2, I2, v, m2, n2);
   }
 #ifdef F2D_PHASE_STAMPS
   __syncthreads();
@@ -3140,13 +3094,13 @@ struct Batch {
   size_t coarse_budget = 0;    // LDS bytes for k_coarse (0: device maximum)
 };
 
-// launches of the fused down-leg of at most this many tiles run the staged
-// 1024-thread form (two workgroups per CU: 512 tiles of 64 x 8 on the 512^2
-// level take 0.8 % less per 1024^2 step than 256 tiles of 64 x 16)
-constexpr double RR_STAGE_TILES_B = 512.;
-// the smallest fused down-leg launches (at most this many tiles of 4 rows:
-// the 128^2 and 64^2 levels at 1024^2) take tiles of 2 fine rows, twice the
-// workgroups, each with half the cells (-0.6 % per 1024^2 step)
+// Tile rows of the fused down-leg: taller tiles (up to 16 fine rows) where
+// those bring the launch to at most this many (two workgroups per CU; taller
+// tiles recompute less overlap): per 4 steps of 1024^2, 6117 us at 512, 6204 at
+// 256, 6242 at 1024, and of 2048 x 1024 Boussinesq 4292, 4416, 4337;
+constexpr double RR_TILES = 512.;
+// and tiles of 2 fine rows on launches of at most this many tiles of 4 (the
+// 128^2 and 64^2 levels): 6117 us at 64, 6143 at 256
 constexpr double RR_SMALL_TILES = 64.;
 // Default of a fine phase's least workgroup count (four per CU).  Tall tiles
 // on a small phase leave the chip idle: 8 x 256^2 FP64, per 4 steps, 4765 us
@@ -3259,7 +3213,7 @@ struct Builder {
   }
   // tile rows of a fused down-leg phase: 2 on the smallest phases, else ty,
   // or the lowest of 8 and `most` (rows) that brings the phase to at most
-  // RR_STAGE_TILES_B tiles
+  // RR_TILES tiles
   int rr_tile_rows(const std::vector<int>& who, const std::vector<int>& start, int dd, int ty,
                    int most) const {
     double cells = 0.;
@@ -3270,9 +3224,9 @@ struct Builder {
       cells += (double)(L.m - 2 * NH) * (L.n - 2 * NH);
     }
     if (cells / ((double)TX * 4) <= RR_SMALL_TILES) return 2;
-    if (cells / ((double)TX * ty) <= RR_STAGE_TILES_B) return ty;
+    if (cells / ((double)TX * ty) <= RR_TILES) return ty;
     for (int t = 2 * ty; t <= most; t *= 2)
-      if (cells / ((double)TX * t) <= RR_STAGE_TILES_B) return t;
+      if (cells / ((double)TX * t) <= RR_TILES) return t;
     return ty;
   }
   int pick_ty(const std::vector<int>& who, const std::vector<int>& start, int dd) const {
@@ -3399,8 +3353,7 @@ struct Builder {
     for (int dd = Dmax; dd >= 0; dd--) {
       const int ty = pick_ty(who, start, dd);
       // the fused down-leg takes taller tiles where that brings its launch
-      // to at most RR_STAGE_TILES tiles (at most two 1024-thread workgroups
-      // per CU, operator staged in LDS); x0 = I(xc) tiles stay at most 8 rows
+      // to at most RR_TILES tiles; x0 = I(xc) tiles stay at most 8 rows
       const int tyr1 = rr_tile_rows(who, start, dd, ty, 16), tyr3 = rr_tile_rows(who, start, dd, ty, 8);
       std::vector<Task> ts, rs, fs, f3;
       for (int i : who) {
@@ -4112,8 +4065,6 @@ static void launch_rr(int ty, unsigned g, hipStream_t s, const Task* TK, const I
                        pred, flags, partial);
 }
 
-constexpr unsigned RR_STAGE_TILES = 512;
-
 template <typename T>
 static int run_prog_t(Batch& b, const std::vector<Launch>& prog, ProfSel* prof = nullptr) {
   const dim3 B2(64, 4), B1(256);
@@ -4241,50 +4192,29 @@ static int run_prog_t(Batch& b, const std::vector<Launch>& prog, ProfSel* prof =
         F2D_LAUNCH(k_gate, dim3((b.ninst + 255) / 256), B1, 0, b.s, b.dD, b.ninst);
         break;
       case L_SMOOTH_RR: {
-        // launches of at most RR_STAGE_TILES workgroups (two per CU or less)
-        // run 1024-thread workgroups and stage the operator in LDS
-        const bool st = g <= RR_STAGE_TILES;
-        const dim3 B16(64, 16);
+        const auto blk = [](int ty2) { return dim3(64, rr_threads(ty2) / 64); };
         if (L.mode == 3) {  // x0 = I(xc): tiles of at most 4 coarse rows
           if (L.ty == 2)
-            F2D_LAUNCH((k_smooth_rr<T, 1, 3, 1, 1024>), dim3(g), B16, 0, b.s, TK, b.dI, Q, b.B,
-                       b.dD, L.pred);
-          else if (L.ty == 4 && st)
-            F2D_LAUNCH((k_smooth_rr<T, 2, 3, 1, 1024>), dim3(g), B16, 0, b.s, TK, b.dI, Q, b.B,
-                       b.dD, L.pred);
-          else if (L.ty == 4)
-            F2D_LAUNCH((k_smooth_rr<T, 2, 3>), dim3(g), B2, 0, b.s, TK, b.dI, Q, b.B, b.dD,
+            F2D_LAUNCH((k_smooth_rr<T, 1, 3>), dim3(g), blk(1), 0, b.s, TK, b.dI, Q, b.B, b.dD,
                        L.pred);
-          else if (st)
-            F2D_LAUNCH((k_smooth_rr<T, 4, 3, 1, 1024>), dim3(g), B16, 0, b.s, TK, b.dI, Q, b.B,
-                       b.dD, L.pred);
+          else if (L.ty == 4)
+            F2D_LAUNCH((k_smooth_rr<T, 2, 3>), dim3(g), blk(2), 0, b.s, TK, b.dI, Q, b.B, b.dD,
+                       L.pred);
           else
-            F2D_LAUNCH((k_smooth_rr<T, 4, 3>), dim3(g), B2, 0, b.s, TK, b.dI, Q, b.B, b.dD,
+            F2D_LAUNCH((k_smooth_rr<T, 4, 3>), dim3(g), blk(4), 0, b.s, TK, b.dI, Q, b.B, b.dD,
                        L.pred);
         } else if (L.ty == 2) {
-          F2D_LAUNCH((k_smooth_rr<T, 1, 1, 1, 1024>), dim3(g), B16, 0, b.s, TK, b.dI, Q, b.B,
-                     b.dD, L.pred);
+          F2D_LAUNCH((k_smooth_rr<T, 1, 1>), dim3(g), blk(1), 0, b.s, TK, b.dI, Q, b.B, b.dD,
+                     L.pred);
         } else if (L.ty == 4) {
-          if (st)
-            F2D_LAUNCH((k_smooth_rr<T, 2, 1, 1, 1024>), dim3(g), B16, 0, b.s, TK, b.dI, Q, b.B,
-                       b.dD, L.pred);
-          else
-            F2D_LAUNCH((k_smooth_rr<T, 2, 1>), dim3(g), B2, 0, b.s, TK, b.dI, Q, b.B, b.dD,
-                       L.pred);
+          F2D_LAUNCH((k_smooth_rr<T, 2, 1>), dim3(g), blk(2), 0, b.s, TK, b.dI, Q, b.B, b.dD,
+                     L.pred);
         } else if (L.ty == 8) {
-          if (st)
-            F2D_LAUNCH((k_smooth_rr<T, 4, 1, 1, 1024>), dim3(g), B16, 0, b.s, TK, b.dI, Q, b.B,
-                       b.dD, L.pred);
-          else
-            F2D_LAUNCH((k_smooth_rr<T, 4, 1>), dim3(g), B2, 0, b.s, TK, b.dI, Q, b.B, b.dD,
-                       L.pred);
+          F2D_LAUNCH((k_smooth_rr<T, 4, 1>), dim3(g), blk(4), 0, b.s, TK, b.dI, Q, b.B, b.dD,
+                     L.pred);
         } else {
-          if (st)
-            F2D_LAUNCH((k_smooth_rr<T, TY2, 1, 1, 1024>), dim3(g), B16, 0, b.s, TK, b.dI, Q, b.B,
-                       b.dD, L.pred);
-          else
-            F2D_LAUNCH((k_smooth_rr<T, TY2, 1>), dim3(g), B2, 0, b.s, TK, b.dI, Q, b.B, b.dD,
-                       L.pred);
+          F2D_LAUNCH((k_smooth_rr<T, TY2, 1>), dim3(g), blk(TY2), 0, b.s, TK, b.dI, Q, b.B, b.dD,
+                     L.pred);
         }
         break;
       }
