@@ -79,6 +79,15 @@ __device__ __forceinline__ int block_all4(bool p) {
   return wf[0] & wf[1] & wf[2] & wf[3];
 }
 
+// the same of two predicates: bits 0 and 1
+__device__ __forceinline__ int block_all4_2(bool p, bool q) {
+  __shared__ int wf[4];
+  const int w = (__all(p) ? 1 : 0) | (__all(q) ? 2 : 0);
+  if (threadIdx.x == 0) wf[threadIdx.y] = w;
+  __syncthreads();
+  return wf[0] & wf[1] & wf[2] & wf[3];
+}
+
 // Step gate (first launch of a step): an instance runs this step while its
 // step budget lasts; every kernel of the step skips instances that do not.
 __global__ void k_gate(DynD* dyn, int ninst) {
@@ -426,6 +435,34 @@ __global__ void __launch_bounds__(256) k_c2c(const Task* __restrict__ tasks,
   }
 }
 
+// A cell's operator row in registers: the eight couplings offdiag_2d reads
+// and the centre A_5 (residual_2d); the arguments are literals after
+// inlining
+template <typename T>
+struct ARow {
+  T a0, a1, a2, a3, a4, a3e, a2s, a1s, a0s;
+  __device__ __forceinline__ T operator()(int k, int dj, int di) const {
+    if (dj == 0 && di == 0)
+      return k == 0 ? a0 : (k == 1 ? a1 : (k == 2 ? a2 : (k == 3 ? a3 : a4)));
+    return k == 3 ? a3e : (k == 2 ? a2s : (k == 1 ? a1s : a0s));
+  }
+};
+// the row of the cell at element e of a level's five planes (PL values each,
+// row length n), every load at once
+template <typename T>
+__device__ __forceinline__ void load_row(ARow<T>& r, const T* A, uint32_t PL, uint32_t n,
+                                         uint32_t e) {
+  r.a4 = ld32(A, 4 * PL + e);
+  r.a0 = ld32(A, e);
+  r.a1 = ld32(A, PL + e);
+  r.a2 = ld32(A, 2 * PL + e);
+  r.a3 = ld32(A, 3 * PL + e);
+  r.a3e = ld32(A, 3 * PL + e + 1);
+  r.a2s = ld32(A, 2 * PL + e + n - 1);
+  r.a1s = ld32(A, PL + e + n);
+  r.a0s = ld32(A, e + n + 1);
+}
+
 // ---------------------------------------------------------------------------
 // k_smooth: two damped-Jacobi sweeps + fill, LDS tile.
 // MODE 0: x = xin; 1: x = 0; 2: x = xin + I(xc); 3: x = I(xc).
@@ -434,6 +471,21 @@ __global__ void __launch_bounds__(256) k_c2c(const Task* __restrict__ tasks,
 // One tile (task ti of `tasks`) of a (64, 4) workgroup; the kernel k_smooth
 // below runs one tile per workgroup, the persistent kernel k_persist any
 // number of them one after another.
+//
+// Block (64, 4).  A thread owns a strip of TYV / 4 consecutive rows of one
+// tile column through both sweeps, with its rhs, mask and (explicit
+// operator) row in registers, and at most one position of the ring around
+// the tile that only the first sweep evaluates.  One memory round trip (every
+// load is issued before the first use), and a sweep reads 3 (R + 2) - R
+// values of LDS for R cells instead of 9 R.
+// What bounds it: the latency of its phases where one round of workgroups
+// holds the launch (1024^2: 4 per compute unit), the rounds themselves
+// beyond that.  Launch bounds that fit one more workgroup spill and lose
+// (2048 x 1024 in 8-row tiles at 64 registers 23.1 us, at 74 17.5).
+// With threads on every fourth row, the right-hand side in LDS and the
+// operator read by each sweep: 1024^2 12.5 us, now 10.6; 2048 x 1024 18.4,
+// now 17.5; explicit 1024 x 512 13.2, now 11.8; whole steps of 1024^2 1535,
+// now 1497 us.
 // Phase timestamps of the 64 x 16 smoother tiles (profiling build only,
 // make stamps): thread 0 of each of the first 2048 workgroups of a launch
 // records the real-time clock (100 MHz) at the start, after the tile loads
@@ -466,25 +518,29 @@ __device__ unsigned long long smooth_stamps[2048 * 8];
 // at every position stored -- x0 += x (hierarchy.py:171) folded into the
 // last smoothing of a refinement V-cycle (no tile of the launch reads that
 // plane); a separate instantiation, so the other smoothings carry none of
-// its code.
-template <typename T, int TYV, bool ADD = false>
+// its code.  BITS: every task of the launch has stencil bits (the finest
+// level), which leaves out the explicit operator's registers (FP64 16 rows:
+// 111 instead of 178).
+template <typename T, int TYV, bool ADD = false, bool BITS = false>
 __device__ __forceinline__ void smooth_tile(const Task* __restrict__ tasks, const int ti,
                                             const InstD* __restrict__ I, T* Q, double* P,
                                             const int8_t* __restrict__ B,
                                             const DynD* __restrict__ dyn, int pred) {
-  // Block (64, 4).  Each phase first issues the global loads of all its
-  // iterations (compile-time trip counts, clamped in-bounds addresses, no
-  // branch between the loads), then computes: one memory round trip per
-  // phase instead of one per iteration.
   constexpr int NT = 256;
   constexpr int XW = TX + 4, XH = TYV + 4, JW = TX + 2, JH = TYV + 2;
-  constexpr int N1 = XH * XW, IT1 = (N1 + NT - 1) / NT;
-  constexpr int N2 = JH * JW, IT2 = (N2 + NT - 1) / NT;
-  constexpr int IT3 = TYV / 4;
+  constexpr int R = TYV / 4;  // rows of a thread's strip
+  // positions around the strips: one ring of the first sweep's region, two
+  // of x's
+  constexpr int NR = 2 * JW + 2 * TYV, NX = 4 * XW + 4 * TYV, ITX = (NX + NT - 1) / NT;
+  static_assert(NR <= NT, "one ring position per thread");
+  // the strips' operator rows stay in registers through both sweeps, except
+  // in the 16-row FP64 tiles, where they alone would take 72 (FP32 ensemble
+  // in 16-row tiles: 16.0 us held, 17.7 read by each sweep)
+  constexpr bool HOLD = R * sizeof(T) <= 16;
   __shared__ T xs[XH][XW];
   __shared__ T j1[JH][JW];
-  __shared__ T bs[JH][JW];         // right-hand side on the first sweep's region
-  __shared__ uint8_t sbs[XH][XW];  // stencil bits (finest level)
+  // stencil bits (finest level); else bit 4 alone: the mask is above 0
+  __shared__ uint8_t sbs[XH][XW];
   F2D_STAMP(0);
   const Task tk = tasks[ti];
   // the skip test is read and taken after the tile loads are issued (the
@@ -498,53 +554,60 @@ __device__ __forceinline__ void smooth_tile(const Task* __restrict__ tasks, cons
   const int final_mask = tk.flags & 1;
   const InstD& in = I[tk.inst];
   const int m = tk.m, n = tk.n;
-  const size_t PL = (size_t)m * n;
+  const uint32_t PL = (uint32_t)m * (uint32_t)n;
   const int8_t* msk = B + tk.msk;
   const T* A = Q + tk.A;
   const T* b = Q + tk.b;
   const T* xin = Q + tk.xin;
-  const int tid = threadIdx.y * 64 + threadIdx.x;
+  const int tx = threadIdx.x, tid = threadIdx.y * 64 + threadIdx.x;
+  const int ty = __builtin_amdgcn_readfirstlane(threadIdx.y);  // one row of threads a wavefront
   const int y0 = tk.y0, x0 = tk.x0;
-  const bool fly = tk.sb >= 0;
+  const bool fly = BITS || tk.sb >= 0;
   const uint8_t* sb = (const uint8_t*)(B + (fly ? tk.sb : 0));
   const bool rdx = MODE == 0 || MODE == 2, rdi = MODE == 2 || MODE == 3;
-  struct {
-    int m, n;
-  } C = {tk.m2, tk.n2};
   const int8_t* msk2 = B + tk.msk2;
   const T* xc = Q + tk.xc;
-  int full_tile = 0;
-  // One round trip: every global load of the tile is issued before the
-  // first is used -- the right-hand side of both sweeps, x and the stencil
-  // bits on the first sweep's stencil region, and for a prolongation the
-  // fine mask there and the coarse tile under it.
-  //
-  // Two forms of the same computation.  The general form maps thread t to
-  // the flat region positions t, t + 256, ... and clips them to the array.
-  // The unclipped form serves tiles whose x region lies inside the array
-  // (every tile of a grid that the tile size divides): thread (x, y) holds
-  // column x of the rows y, y + 4, ..., the four (x region) or two
-  // (first-sweep region) columns past the 64th go to the first threads of
-  // the block, and every offset is the thread's base plus a multiple of
-  // four rows -- no division, bounds test or select per element.
-  constexpr int KX = XH / 4, KB = (JH + 3) / 4;
-  static_assert(XH % 4 == 0 && KB <= IT2 && KX + 1 <= IT1, "unclipped form registers");
+  const int rows = ty * R;  // first tile row of the strip
+  // a tile whose x region lies inside the array is not clipped
   const bool lean = y0 + TYV + 1 <= m - 2 && x0 + TX + 1 <= n - 2;
-  const int tx = threadIdx.x, ty = threadIdx.y;
-  const uint32_t s4 = 4u * (uint32_t)n;
-  const uint32_t ox = at32(y0 - 2 + ty, x0 - 2 + tx, n);  // x region (ty, tx)
-  const uint32_t ob = ox + (uint32_t)n + 1u;              // first-sweep region (ty, tx)
-  const bool xe_on = tid < 4 * XH, be_on = tid < 2 * JH;
-  const int xer = xe_on ? tid >> 2 : 0, xec = TX + (tid & 3);
-  const int ber = be_on ? tid >> 1 : 0, bec = TX + (tid & 1);
-  const uint32_t oxe = at32(y0 - 2 + xer, x0 - 2 + xec, n);
-  const uint32_t obe = at32(y0 - 1 + ber, x0 - 1 + bec, n);
-  uint32_t cc2[IT2];
-  bool ok2[IT2];
-  T bv[IT2];
-  T be = T(0);
+  const uint32_t safe = at32(NH, NH, n);
+  const uint32_t o0 = at32(y0 + rows, x0 + tx, n);
+  // first-sweep position (rr, cc) of this thread on the ring
+  int rr1, cc1;
+  {
+    const int e = tid - 2 * JW;
+    rr1 = tid < JW ? 0 : (e < 0 ? JH - 1 : 1 + (e >> 1));
+    cc1 = tid < JW ? tid : (e < 0 ? tid - JW : (e & 1) * (JW - 1));
+  }
+  const bool on1 = tid < NR;
+  const bool ok1 = on1 && (lean || (y0 - 1 + rr1 <= m - NH && x0 - 1 + cc1 <= n - NH));
+  const uint32_t o1 = ok1 ? at32(y0 - 1 + rr1, x0 - 1 + cc1, n) : safe;
+  int rrx[ITX], ccx[ITX];
+  bool onx[ITX], okx[ITX];
+  uint32_t ox[ITX];
+#pragma unroll
+  for (int it = 0; it < ITX; it++) {
+    const int q = tid + it * NT, a = q / XW, e = q - 4 * XW, s = e & 3;
+    rrx[it] = e < 0 ? (a < 2 ? a : XH - 4 + a) : 2 + (e >> 2);
+    ccx[it] = e < 0 ? q - a * XW : (s < 2 ? s : XW - 4 + s);
+    onx[it] = q < NX;
+    okx[it] = onx[it] && (lean || (y0 - 2 + rrx[it] <= m - 2 && x0 - 2 + ccx[it] <= n - 2));
+    ox[it] = okx[it] ? at32(y0 - 2 + rrx[it], x0 - 2 + ccx[it], n) : safe;
+  }
+  // strip cell k: inside the x region's clip, and inside the first sweep's
+  bool okm[R], ok2[R];
+  uint32_t om[R];
+#pragma unroll
+  for (int k = 0; k < R; k++) {
+    const int J = y0 + rows + k, Ii = x0 + tx;
+    okm[k] = lean || (J <= m - 2 && Ii <= n - 2);
+    ok2[k] = lean || (J <= m - NH && Ii <= n - NH);
+    om[k] = okm[k] ? o0 + (uint32_t)k * (uint32_t)n : safe;
+  }
   // the plane the stored values are added to (task flag 4), and its values
-  // at the tile's cells in the unclipped form, loaded with the tile
+  // at the strip of a tile without images, loaded with the tile
+  const bool noimg =
+      y0 >= 2 * NH && y0 + TYV <= m - 2 * NH && x0 >= 2 * NH && x0 + TX <= n - 2 * NH;
   const bool addp = ADD && (tk.flags & 4) != 0;
   double* pw = nullptr;
   if constexpr (sizeof(T) == 8) {
@@ -552,112 +615,87 @@ __device__ __forceinline__ void smooth_tile(const Task* __restrict__ tasks, cons
   } else {
     pw = addp ? P + tk.xcc : nullptr;
   }
-  double pv[IT3];
-  if (lean) {
+  // one round trip: every load of the tile before the first use
+  T xv[R], xr[ITX], bv[R], be;
+  double pv[R];
+  uint8_t bt[R], btx[ITX];
+  int8_t mv[R], mx[ITX], me = 0;
+  ARow<T> row[R], rowe;
 #pragma unroll
-    for (int k = 0; k < KB; k++) bv[k] = ld32(b, ty + 4 * k < JH ? ob + k * s4 : ob);
-    be = ld32(b, obe);
-    if (addp) {
+  for (int k = 0; k < R; k++) xv[k] = rdx ? ld32(xin, om[k]) : T(0);
 #pragma unroll
-      for (int k = 0; k < IT3; k++) pv[k] = ld32(pw, ob + (uint32_t)n + 1u + k * s4);
-    }
+  for (int it = 0; it < ITX; it++) xr[it] = rdx ? ld32(xin, ox[it]) : T(0);
+  if (fly) {
+#pragma unroll
+    for (int k = 0; k < R; k++) bt[k] = ld32(sb, om[k]);
+#pragma unroll
+    for (int it = 0; it < ITX; it++) btx[it] = ld32(sb, ox[it]);
   } else {
 #pragma unroll
-    for (int it = 0; it < IT2; it++) {
-      const int q = tid + it * NT;
-      const int rr = q / JW, cc = q - rr * JW;
-      const int j = y0 - 1 + rr, i = x0 - 1 + cc;
-      ok2[it] = q < N2 && j <= m - NH && i <= n - NH;
-      cc2[it] = ok2[it] ? at32(j, i, n) : 0u;
-    }
+    for (int k = 0; k < R; k++) mv[k] = ld32(msk, om[k]);
 #pragma unroll
-    for (int it = 0; it < IT2; it++) bv[it] = ld32(b, cc2[it]);
+    for (int it = 0; it < ITX; it++) mx[it] = ld32(msk, ox[it]);
   }
-  const int Ic = x0 + threadIdx.x;
-  // x region: rows [y0-2, y0+TY+1] x cols [x0-2, x0+TX+1], clipped to
-  // [1, m-2]; the coarse points its prolongation reads are rows
-  // [y0>>1, +CH) x cols [x0>>1, +CW) (clamped to the coarse array)
+#pragma unroll
+  for (int k = 0; k < R; k++) bv[k] = ld32(b, ok2[k] ? om[k] : safe);
+  be = ld32(b, o1);
+  if (ADD && addp && noimg) {
+#pragma unroll
+    for (int k = 0; k < R; k++) pv[k] = ld32(pw, om[k]);
+  }
+  // the coarse tile under the x region (rows [y0>>1, +CH) x cols
+  // [x0>>1, +CW), clamped to the coarse array)
   constexpr int CH = TYV / 2 + 4, CW = TX / 2 + 4, NC = CH * CW, ITC = (NC + NT - 1) / NT;
   __shared__ T cxs[CH][CW];
   __shared__ int8_t cms[CH][CW];
-  __shared__ int8_t ms1[XH][XW];  // fine mask of the prolongation
   const int cy0 = y0 >> 1, cx0 = x0 >> 1;
-  bool ok1[IT1];
-  T xv[IT1];
-  uint8_t bt[IT1];
-  int8_t m1v[IT1];
   T cxv[ITC];
   int8_t cmv[ITC];
-  // the fine mask of the prolongation: bit 4 of the stencil bits where
-  // they exist (the level's 0/1 mask), else loaded
-  if (lean) {
-#pragma unroll
-    for (int k = 0; k <= KX; k++) {  // rows ty + 4k, then the extra columns
-      const uint32_t c = k < KX ? ox + k * s4 : oxe;
-      xv[k] = rdx ? ld32(xin, c) : T(0);
-      bt[k] = fly ? ld32(sb, c) : (uint8_t)0;
-      m1v[k] = (rdi && !fly) ? ld32(msk, c) : (int8_t)0;
-    }
-  } else {
-#pragma unroll
-    for (int it = 0; it < IT1; it++) {
-      const int q = tid + it * NT;
-      const int rr = q / XW, cc = q - rr * XW;
-      const int j = y0 - 2 + rr, i = x0 - 2 + cc;
-      ok1[it] = q < N1 && j <= m - 2 && i <= n - 2;
-      const uint32_t c = ok1[it] ? at32(j, i, n) : at32(1, 1, n);
-      xv[it] = rdx ? ld32(xin, c) : T(0);
-      bt[it] = fly ? ld32(sb, c) : (uint8_t)0;
-      m1v[it] = (rdi && !fly) ? ld32(msk, c) : (int8_t)0;
-    }
-  }
   if (rdi) {
 #pragma unroll
     for (int it = 0; it < ITC; it++) {
       const int q = min(tid + it * NT, NC - 1);
       const int rr = q / CW, cc = q - rr * CW;
-      const uint32_t c = at32(min(cy0 + rr, C.m - 1), min(cx0 + cc, C.n - 1), C.n);
+      const uint32_t c = at32(min(cy0 + rr, tk.m2 - 1), min(cx0 + cc, tk.n2 - 1), tk.n2);
       cxv[it] = ld32(xc, c);
       cmv[it] = ld32(msk2, c);
     }
   }
+  if (!fly) {
+    me = ld32(msk, o1);
+    if constexpr (HOLD) {
+#pragma unroll
+      for (int k = 0; k < R; k++) load_row(row[k], A, PL, (uint32_t)n, ok2[k] ? om[k] : safe);
+    }
+    if constexpr (HOLD) load_row(rowe, A, PL, (uint32_t)n, o1);
+  }
   if (skip(dyn, tk.inst, pred)) return;
   F2D_STAMP(1);
-  bool full = true;
-  if (lean) {
+  // bit 0 of `all`: every cell of the x region has the full 9-point stencil;
+  // bit 1: it and the coarse tile are fluid (weights of the prolongation)
+  bool full = true, fluid = true;
 #pragma unroll
-    for (int k = 0; k < KB; k++)
-      if (ty + 4 * k < JH) bs[ty + 4 * k][tx] = bv[k];
-    if (be_on) bs[ber][bec] = be;
+  for (int k = 0; k < R; k++) {
+    if (fly)
+      mv[k] = (int8_t)((bt[k] >> 4) & 1);
+    else
+      bt[k] = mv[k] > 0 ? 16 : 0;
+    sbs[rows + k + 2][tx + 2] = okm[k] ? bt[k] : (uint8_t)0;
+    xv[k] = okm[k] ? xv[k] : T(0);
+    full = full && okm[k] && bt[k] == 31;
+    fluid = fluid && okm[k] && mv[k] == 1;
+  }
 #pragma unroll
-    for (int k = 0; k <= KX; k++) {
-      if (k == KX && !xe_on) continue;
-      const int rr = k < KX ? ty + 4 * k : xer, cc = k < KX ? tx : xec;
-      xs[rr][cc] = xv[k];
-      sbs[rr][cc] = bt[k];
-      ms1[rr][cc] = fly ? (int8_t)((bt[k] >> 4) & 1) : m1v[k];
-      full = full && bt[k] == 31;
-    }
-  } else {
-#pragma unroll
-    for (int it = 0; it < IT2; it++) {
-      const int q = tid + it * NT;
-      if (q < N2) {
-        const int rr = q / JW, cc = q - rr * JW;
-        bs[rr][cc] = ok2[it] ? bv[it] : T(0);
-      }
-    }
-#pragma unroll
-    for (int it = 0; it < IT1; it++) {
-      const int q = tid + it * NT;
-      if (q < N1) {
-        const int rr = q / XW, cc = q - rr * XW;
-        xs[rr][cc] = ok1[it] ? xv[it] : T(0);
-        sbs[rr][cc] = ok1[it] ? bt[it] : (uint8_t)0;
-        ms1[rr][cc] = fly ? (int8_t)((bt[it] >> 4) & 1) : m1v[it];
-        full = full && ok1[it] && bt[it] == 31;
-      }
-    }
+  for (int it = 0; it < ITX; it++) {
+    if (!onx[it]) continue;
+    if (fly)
+      mx[it] = (int8_t)((btx[it] >> 4) & 1);
+    else
+      btx[it] = mx[it] > 0 ? 16 : 0;
+    sbs[rrx[it]][ccx[it]] = okx[it] ? btx[it] : (uint8_t)0;
+    xr[it] = okx[it] ? xr[it] : T(0);
+    full = full && okx[it] && btx[it] == 31;
+    fluid = fluid && okx[it] && mx[it] == 1;
   }
   if (rdi) {
 #pragma unroll
@@ -667,165 +705,182 @@ __device__ __forceinline__ void smooth_tile(const Task* __restrict__ tasks, cons
         const int rr = q / CW, cc = q - rr * CW;
         cxs[rr][cc] = cxv[it];
         cms[rr][cc] = cmv[it];
+        fluid = fluid && cmv[it] == 1;
       }
     }
-    __syncthreads();
-    // prolongation (ip_eval: interp_at's expressions) of the coarse tile,
-    // added to x (MODE 2) or replacing it (MODE 3).  Work goes by coarse
-    // cell: coarse (J2, I2) and its right/lower neighbours give the four
-    // fine points (2 J2 - 2 + dj, 2 I2 - 2 + di), whose parities are
-    // (dj, di), so the operands are read once for four points.
-    constexpr int CRH = XH / 2 + 1, CRW = XW / 2 + 1, NCR = CRH * CRW;
+  }
+  auto put_x = [&]() {
 #pragma unroll
-    for (int it = 0; it < (NCR + NT - 1) / NT; it++) {
-      const int q = tid + it * NT;
-      if (q >= NCR) continue;
-      const int a = q / CRW, bc = q - a * CRW;
-      IpOps<T> o;
-      o.a = cxs[a][bc];
-      o.b = cxs[a][bc + 1];
-      o.c = cxs[a + 1][bc];
-      o.d = cxs[a + 1][bc + 1];
-      o.sa = cms[a][bc];
-      o.sb = cms[a][bc + 1];
-      o.sc = cms[a + 1][bc];
-      o.sd = cms[a + 1][bc + 1];
+    for (int k = 0; k < R; k++) xs[rows + k + 2][tx + 2] = xv[k];
 #pragma unroll
-      for (int dj = 0; dj < 2; dj++)
+    for (int it = 0; it < ITX; it++)
+      if (onx[it]) xs[rrx[it]][ccx[it]] = xr[it];
+  };
+  put_x();
+  const int all = block_all4_2(fly && full, fluid);
+  F2D_STAMP(2);
+  if (rdi) {
+    // the prolongation (interp_at's expressions) of the coarse tile, added
+    // to x (MODE 2) or replacing it (MODE 3)
+    if (all & 2) {
+      // all masks 1: the weights are 1, 1/2, 1/2, 1/4
+      auto ip = [&](int rr, int cc) {
+        const int a = ((y0 + rr) >> 1) - cy0, c = ((x0 + cc) >> 1) - cx0;
+        const bool pi = ((x0 + cc) & 1) != 0;
+        const T va = cxs[a][c], vb = cxs[a][c + 1];
+        if (((y0 + rr) & 1) == 0) return pi ? (va + vb) * T(0.5) : va;
+        const T vc = cxs[a + 1][c], vd = cxs[a + 1][c + 1];
+        return pi ? T(0.25) * (va + vb + vc + vd) : (va + vc) * T(0.5);
+      };
 #pragma unroll
-        for (int di = 0; di < 2; di++) {
-          const int j = 2 * (cy0 + a) - 2 + dj, i = 2 * (cx0 + bc) - 2 + di;
-          const int rr = j - (y0 - 2), cc = i - (x0 - 2);
-          if (rr < 0 || rr >= XH || cc < 0 || cc >= XW || j > m - 2 || i > n - 2) continue;
-          o.m1 = ms1[rr][cc];
-          o.par = di | (dj << 1);
-          const T r = ip_eval<T>(o);
-          xs[rr][cc] = MODE == 2 ? xs[rr][cc] + r : r;
-        }
+      for (int k = 0; k < R; k++) {
+        const T r = ip(rows + k + 2, tx + 2);
+        xv[k] = MODE == 2 ? xv[k] + r : r;
+      }
+#pragma unroll
+      for (int it = 0; it < ITX; it++) {
+        if (!onx[it]) continue;
+        const T r = ip(rrx[it], ccx[it]);
+        xr[it] = MODE == 2 ? xr[it] + r : r;
+      }
+      put_x();
+      __syncthreads();
+    } else {
+      // by coarse cell: (J2, I2) and its right/lower neighbours give the
+      // four fine points (2 J2 - 2 + dj, 2 I2 - 2 + di), whose parities are
+      // (dj, di), so the operands and masks are read once for four points
+      constexpr int CRH = XH / 2 + 1, CRW = XW / 2 + 1, NCR = CRH * CRW;
+#pragma unroll
+      for (int it = 0; it < (NCR + NT - 1) / NT; it++) {
+        const int q = tid + it * NT;
+        if (q >= NCR) continue;
+        const int a = q / CRW, bc = q - a * CRW;
+        IpOps<T> o;
+        o.a = cxs[a][bc];
+        o.b = cxs[a][bc + 1];
+        o.c = cxs[a + 1][bc];
+        o.d = cxs[a + 1][bc + 1];
+        o.sa = cms[a][bc];
+        o.sb = cms[a][bc + 1];
+        o.sc = cms[a + 1][bc];
+        o.sd = cms[a + 1][bc + 1];
+#pragma unroll
+        for (int dj = 0; dj < 2; dj++)
+#pragma unroll
+          for (int di = 0; di < 2; di++) {
+            const int j = 2 * (cy0 + a) - 2 + dj, i = 2 * (cx0 + bc) - 2 + di;
+            const int rr = j - (y0 - 2), cc = i - (x0 - 2);
+            if (rr < 0 || rr >= XH || cc < 0 || cc >= XW || j > m - 2 || i > n - 2) continue;
+            o.m1 = (int8_t)(sbs[rr][cc] & 16);
+            o.par = di | (dj << 1);
+            const T r = ip_eval<T>(o);
+            xs[rr][cc] = MODE == 2 ? xs[rr][cc] + r : r;
+          }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < R; k++) xv[k] = xs[rows + k + 2][tx + 2];
     }
   }
-  // every cell of the tile has the full 9-point stencil: constant weights
-  F2D_STAMP_SYNC(2);
-  full_tile = block_all4(fly && full);
   F2D_STAMP(3);
   const T c1 = T(in.omega), c2 = T(1. - in.omega);
   T* xout = Q + tk.xout;
   const int8_t* mp = final_mask ? B + in.mskp : nullptr;
   T w[5];
   for (int k = 0; k < 5; k++) w[k] = T(in.w0[k]);
-  // the plane += the value stored at interior (J, I) and at each image
-  auto add_img = [&](int J, int I, T v) {
-    each_img(J, I, m, n, [&](int j, int i) {
-      const uint32_t c = at32(j, i, n);
-      const T sv = mp ? v * T(ld32(mp, c)) : v;
-      st32(pw, c, ld32(pw, c) + (double)sv);
+  // one sweep of the strip: t points at its first cell in a tile of rows of
+  // W values, v the strip's own values there; jac(k, X) relaxes cell k
+  auto strip = [&](const auto* t, const int W, const T* v, auto jac, auto out) {
+    T h[R + 2][3];
+#pragma unroll
+    for (int r = 0; r < R + 2; r++)
+#pragma unroll
+      for (int c = 0; c < 3; c++)
+        h[r][c] = c == 1 && r >= 1 && r <= R ? v[r >= 1 && r <= R ? r - 1 : 0]
+                                             : t[(r - 1) * W + c - 1];
+#pragma unroll
+    for (int k = 0; k < R; k++)
+      out(k, jac(k, [&](int dj, int di) { return h[k + 1 + dj][1 + di]; }));
+  };
+  // jm relaxes strip cell k, jr the ring's position
+  auto sweeps = [&](auto jm, auto jr) {
+    T v1[R];
+    strip(&xs[rows + 2][tx + 2], XW, xv, jm, [&](int k, T v) {
+      v1[k] = ok2[k] ? v : T(0);
+      j1[rows + k + 1][tx + 1] = v1[k];
     });
-  };
-  // Jac(c, r, q, b, X): damped-Jacobi value of the cell at global c, tile
-  // (r, q) of the x/bits tiles, right-hand side b, neighbour accessor X
-  auto sweeps = [&](auto Jac) {
-    // phase 2: first sweep on rows [y0-1, y0+TY] x cols [x0-1, x0+TX],
-    // clipped to [.., m-NH]
-    {
-#pragma unroll
-      for (int it = 0; it < IT2; it++) {
-        const int q = tid + it * NT;
-        if (q < N2) {
-          const int rr = q / JW, cc = q - rr * JW;
-          T v = T(0);
-          if (ok2[it]) {
-            const size_t c = cc2[it];
-            v = Jac(c, rr + 1, cc + 1, bv[it],
-                    [&](int dj, int di) { return xs[rr + 1 + dj][cc + 1 + di]; });
-          }
-          j1[rr][cc] = v;
-        }
-      }
+    if (on1) {
+      const T v = jr([&](int dj, int di) { return xs[rr1 + 1 + dj][cc1 + 1 + di]; });
+      j1[rr1][cc1] = ok1 ? v : T(0);
     }
-    __syncthreads();
-    // phase 3: second sweep on the tile interior, stored with its images
-#pragma unroll
-    for (int k = 0; k < IT3; k++) {
-      const int rr = threadIdx.y + 4 * k, cc = threadIdx.x;
-      const int J = y0 + rr;
-      if (J >= m - NH || Ic >= n - NH) continue;
-      const size_t c = at32(J, Ic, n);
-      const T v = Jac(c, rr + 2, cc + 2, bs[rr + 1][cc + 1],
-                      [&](int dj, int di) { return j1[rr + 1 + dj][cc + 1 + di]; });
-      store_img_mask32<T>(xout, mp, J, Ic, v, m, n);
-      if (addp) add_img(J, Ic, v);
-    }
-  };
-  // the same two sweeps in the unclipped form; stores without images when
-  // no cell of the tile has one
-  const bool noimg =
-      y0 >= 2 * NH && y0 + TYV <= m - 2 * NH && x0 >= 2 * NH && x0 + TX <= n - 2 * NH;
-  auto sweeps_lean = [&](auto Jac) {
-#pragma unroll
-    for (int k = 0; k < KB; k++) {
-      const int rr = ty + 4 * k;
-      if (rr < JH)
-        j1[rr][tx] = Jac(ob + k * s4, rr + 1, tx + 1, bv[k],
-                         [&](int dj, int di) { return xs[rr + 1 + dj][tx + 1 + di]; });
-    }
-    if (be_on)
-      j1[ber][bec] = Jac(obe, ber + 1, bec + 1, be,
-                         [&](int dj, int di) { return xs[ber + 1 + dj][bec + 1 + di]; });
     __syncthreads();
     F2D_STAMP(4);
-#pragma unroll
-    for (int k = 0; k < IT3; k++) {
-      const int rr = ty + 4 * k;
-      const uint32_t c = ob + (uint32_t)n + 1u + k * s4;  // (y0 + rr, x0 + tx)
-      const T v = Jac(c, rr + 2, tx + 2, bs[rr + 1][tx + 1],
-                      [&](int dj, int di) { return j1[rr + 1 + dj][tx + 1 + di]; });
+    strip(&j1[rows + 1][tx + 1], JW, v1, jm, [&](int k, T v) {
+      const int J = y0 + rows + k, Ic = x0 + tx;
       if (noimg) {
-        const T sv = mp ? v * T(ld32(mp, c)) : v;
-        st32(xout, c, sv);
-        if (addp) st32(pw, c, pv[k] + (double)sv);
-      } else {
-        store_img_mask32<T>(xout, mp, y0 + rr, Ic, v, m, n);
-        if (addp) add_img(y0 + rr, Ic, v);
+        const T sv = mp ? v * T(ld32(mp, om[k])) : v;
+        st32(xout, om[k], sv);
+        if (ADD && addp) st32(pw, om[k], pv[k] + (double)sv);
+      } else if (J < m - NH && Ic < n - NH) {
+        store_img_mask32<T>(xout, mp, J, Ic, v, m, n);
+        if (ADD && addp)
+          // the plane += the value stored at interior (J, I) and each image
+          each_img(J, Ic, m, n, [&](int j, int i) {
+            const uint32_t c = at32(j, i, n);
+            const T sv = mp ? v * T(ld32(mp, c)) : v;
+            st32(pw, c, ld32(pw, c) + (double)sv);
+          });
       }
-    }
+    });
     F2D_STAMP_SYNC(5);
   };
-  auto run = [&](auto Jac) {
-    if (lean)
-      sweeps_lean(Jac);
-    else
-      sweeps(Jac);
-  };
-  if (full_tile) {
-    // A_k = w_k everywhere, the mask is 1, and c1 / |A_5| is one value
+  if (fly) {
+    // one c1 / |A_5| serves the tile: A_5 = w_5 wherever the mask (bit 4) is
+    // set, and the value is discarded where it is not
     const T c3 = c1 / fabs(w[4]);
-    run([&](size_t, int, int, T bc, auto X) {
-      return jacobi_c3_2d<T>(bc, c3, c2, [&](int k, int, int) { return w[k]; }, X);
-    });
-  } else if (fly) {
-    // A_5 = w_5 wherever the mask (bit 4) is set, and the value is
-    // discarded where it is not: one c1 / |A_5| serves the tile
-    const T c3 = c1 / fabs(w[4]);
-    run([&](size_t, int r, int q, T bc, auto X) {
-      const T v = jacobi_c3_2d<T>(bc, c3, c2, ABitsTile2<T, XW>{&sbs[r][q], w}, X);
-      return bit_select<T>(sbs[r][q], 4, v);
-    });
-  } else {
-    run([&](size_t c, int, int, T bc, auto X) {
-      const APlanes<T> Ap{A, PL, c};
-      return jacobi_2d<T>(msk[c], bc, c1, c2,
-                          [&](int k, int dj, int di) { return Ap(k, (ptrdiff_t)dj * n + di); },
-                          X);
-    });
+    if (all & 1) {
+      // A_k = w_k everywhere and the mask is 1
+      auto wk = [&](int k, int, int) { return w[k]; };
+      sweeps([&](int k, auto X) { return jacobi_c3_2d<T>(bv[k], c3, c2, wk, X); },
+             [&](auto X) { return jacobi_c3_2d<T>(be, c3, c2, wk, X); });
+    } else {
+      auto jac = [&](T bc, int r, int q, auto X) {
+        const T v = jacobi_c3_2d<T>(bc, c3, c2, ABitsTile2<T, XW>{&sbs[r][q], w}, X);
+        return bit_select<T>(sbs[r][q], 4, v);
+      };
+      sweeps([&](int k, auto X) { return jac(bv[k], rows + k + 2, tx + 2, X); },
+             [&](auto X) { return jac(be, rr1 + 1, cc1 + 1, X); });
+    }
+  } else if constexpr (!BITS) {
+    T c3[R];
+    if constexpr (HOLD) {
+#pragma unroll
+      for (int k = 0; k < R; k++) c3[k] = c1 / fabs(row[k].a4);
+    }
+    sweeps(
+        [&](int k, auto X) {
+          if constexpr (HOLD) {
+            const T v = jacobi_c3_2d<T>(bv[k], c3[k], c2, row[k], X);
+            return mv[k] == 0 ? T(0) : v;
+          } else {
+            ARow<T> r;
+            load_row(r, A, PL, (uint32_t)n, ok2[k] ? om[k] : safe);
+            return jacobi_2d<T>(mv[k], bv[k], c1, c2, r, X);
+          }
+        },
+        [&](auto X) {
+          if constexpr (!HOLD) load_row(rowe, A, PL, (uint32_t)n, o1);
+          return jacobi_2d<T>(me, be, c1, c2, rowe, X);
+        });
   }
 }
 
-template <typename T, int TYV, bool ADD = false>
+template <typename T, int TYV, bool ADD = false, bool BITS = false>
 __global__ void __launch_bounds__(256) k_smooth(const Task* __restrict__ tasks,
                                                 const InstD* __restrict__ I, T* Q, double* P,
                                                 const int8_t* __restrict__ B,
                                                 const DynD* __restrict__ dyn, int pred) {
-  smooth_tile<T, TYV, ADD>(tasks, task_index(), I, Q, P, B, dyn, pred);
+  smooth_tile<T, TYV, ADD, BITS>(tasks, task_index(), I, Q, P, B, dyn, pred);
 }
 
 // ---------------------------------------------------------------------------
@@ -1159,34 +1214,6 @@ __global__ void __launch_bounds__(NTH) k_restrict_b2(const Task* __restrict__ ta
       v = restrict_r<T>([&](int dj, int di) { return ms[2 * ry + 1 + dj][2 * rx + 1 + di]; });
     store_img_mask32<T>(bo, nullptr, J, Ii, v, mo, no);
   }
-}
-
-// A cell's operator row in registers: the eight couplings offdiag_2d reads
-// and the centre A_5 (residual_2d); the arguments are literals after
-// inlining
-template <typename T>
-struct ARow {
-  T a0, a1, a2, a3, a4, a3e, a2s, a1s, a0s;
-  __device__ __forceinline__ T operator()(int k, int dj, int di) const {
-    if (dj == 0 && di == 0)
-      return k == 0 ? a0 : (k == 1 ? a1 : (k == 2 ? a2 : (k == 3 ? a3 : a4)));
-    return k == 3 ? a3e : (k == 2 ? a2s : (k == 1 ? a1s : a0s));
-  }
-};
-// the row of the cell at element e of a level's five planes (PL values each,
-// row length n), every load at once
-template <typename T>
-__device__ __forceinline__ void load_row(ARow<T>& r, const T* A, uint32_t PL, uint32_t n,
-                                         uint32_t e) {
-  r.a4 = ld32(A, 4 * PL + e);
-  r.a0 = ld32(A, e);
-  r.a1 = ld32(A, PL + e);
-  r.a2 = ld32(A, 2 * PL + e);
-  r.a3 = ld32(A, 3 * PL + e);
-  r.a3e = ld32(A, 3 * PL + e + 1);
-  r.a2s = ld32(A, 2 * PL + e + n - 1);
-  r.a1s = ld32(A, PL + e + n);
-  r.a0s = ld32(A, e + n + 1);
 }
 
 // ---------------------------------------------------------------------------
@@ -4049,6 +4076,17 @@ struct ProfSel {
 
 #define F2D_LAUNCH(K, G, B, S, STREAM, ...) hipLaunchKernelGGL(K, G, B, S, STREAM, __VA_ARGS__)
 
+template <typename T, bool ADD, bool BITS>
+static void launch_smooth(int ty, unsigned g, hipStream_t s, const Task* TK, const InstD* dI, T* Q,
+                          double* P, const int8_t* B, const DynD* dD, int pred) {
+  const dim3 B2(64, 4);
+  if (ty == 4)
+    F2D_LAUNCH((k_smooth<T, 4, ADD, BITS>), dim3(g), B2, 0, s, TK, dI, Q, P, B, dD, pred);
+  else if (ty == 8)
+    F2D_LAUNCH((k_smooth<T, 8, ADD, BITS>), dim3(g), B2, 0, s, TK, dI, Q, P, B, dD, pred);
+  else
+    F2D_LAUNCH((k_smooth<T, TY, ADD, BITS>), dim3(g), B2, 0, s, TK, dI, Q, P, B, dD, pred);
+}
 template <typename T, typename R>
 static void launch_rr(int ty, unsigned g, hipStream_t s, const Task* TK, const InstD* dI,
                       const R* RP, T* Q, const int8_t* B, const DynD* dD, int pred, int flags,
@@ -4115,23 +4153,16 @@ static int run_prog_t(Batch& b, const std::vector<Launch>& prog, ProfSel* prof =
           F2D_LAUNCH((k_c2c<T, T>), dim3(g), B2, 0, b.s, TK, b.dI, Q, Q, b.dD, L.pred);
         break;
       case L_SMOOTH:
-        // launch flag 16: tasks that add their result to a plane (k_smooth ADD)
-        if ((L.flags & 16) && L.ty == 4)
-          F2D_LAUNCH((k_smooth<T, 4, true>), dim3(g), B2, 0, b.s, TK, b.dI, Q, P, b.B, b.dD,
-                     L.pred);
-        else if ((L.flags & 16) && L.ty == 8)
-          F2D_LAUNCH((k_smooth<T, 8, true>), dim3(g), B2, 0, b.s, TK, b.dI, Q, P, b.B, b.dD,
-                     L.pred);
+        // launch flag 16: tasks that add their result to a plane (k_smooth
+        // ADD); 32: every task has stencil bits (k_smooth BITS)
+        if ((L.flags & 48) == 48)
+          launch_smooth<T, true, true>(L.ty, g, b.s, TK, b.dI, Q, P, b.B, b.dD, L.pred);
         else if (L.flags & 16)
-          F2D_LAUNCH((k_smooth<T, TY, true>), dim3(g), B2, 0, b.s, TK, b.dI, Q, P, b.B, b.dD,
-                     L.pred);
-        else if (L.ty == 4)
-          F2D_LAUNCH((k_smooth<T, 4>), dim3(g), B2, 0, b.s, TK, b.dI, Q, P, b.B, b.dD, L.pred);
-        else if (L.ty == 8)
-          F2D_LAUNCH((k_smooth<T, 8>), dim3(g), B2, 0, b.s, TK, b.dI, Q, P, b.B, b.dD, L.pred);
+          launch_smooth<T, true, false>(L.ty, g, b.s, TK, b.dI, Q, P, b.B, b.dD, L.pred);
+        else if (L.flags & 32)
+          launch_smooth<T, false, true>(L.ty, g, b.s, TK, b.dI, Q, P, b.B, b.dD, L.pred);
         else
-          F2D_LAUNCH((k_smooth<T, TY>), dim3(g), B2, 0, b.s, TK, b.dI, Q, P, b.B, b.dD,
-                             L.pred);
+          launch_smooth<T, false, false>(L.ty, g, b.s, TK, b.dI, Q, P, b.B, b.dD, L.pred);
         break;
       case L_RR:
         if (L.flags & 32)
@@ -4548,9 +4579,9 @@ static int build_programs(Batch& b) {
 // the task tables and reduction scratch of the built programs
 static int upload_programs(Batch& b) {
   size_t np = 0;
-  std::vector<const std::vector<Launch>*> progs = {&b.prog_init, &b.prog_step, &b.prog_diag};
-  for (const auto& po : b.prog_one) progs.push_back(&po);
-  for (const auto& po : b.prog_mom) progs.push_back(&po);
+  std::vector<std::vector<Launch>*> progs = {&b.prog_init, &b.prog_step, &b.prog_diag};
+  for (auto& po : b.prog_one) progs.push_back(&po);
+  for (auto& po : b.prog_mom) progs.push_back(&po);
   for (auto* pr : progs)
     for (const Launch& L : *pr)
       if (L.kind == L_RR || L.kind == L_DIAG || L.kind == L_NSDOT)
@@ -4593,8 +4624,13 @@ static int upload_programs(Batch& b) {
   for (size_t k = 0; k < dev.size(); k++) dev[k].slot = 0;
   std::vector<char> placed(b.tasks.size(), 0);
   for (auto* pr : progs)
-    for (const Launch& L : *pr) {
+    for (Launch& L : *pr) {
       if (L.ntask <= 0 || L.kind == L_FOLD || L.kind == L_GATE || L.kind == L_PERSIST) continue;
+      if (L.kind == L_SMOOTH) {
+        bool bits = true;
+        for (int k = 0; k < L.ntask; k++) bits = bits && b.tasks[L.toff + k].sb >= 0;
+        L.flags = bits ? L.flags | 32 : L.flags & ~32;
+      }
       if (placed[L.toff]) continue;
       for (int k = 0; k < L.ntask; k++) {
         const int src = L.kind == L_COARSE ? k : xcd_task(k, L.ntask);
