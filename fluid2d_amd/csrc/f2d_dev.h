@@ -569,4 +569,32 @@ __device__ __forceinline__ void store_img_mask32(T* a, const int8_t* mk, int J, 
   if (jm && im) put(J - M, I - N);
 }
 
+// A cell's operator row in registers: the eight couplings offdiag_2d reads
+// and the centre A_5 (residual_2d); the arguments are literals after
+// inlining
+template <typename T>
+struct ARow {
+  T a0, a1, a2, a3, a4, a3e, a2s, a1s, a0s;
+  __device__ __forceinline__ T operator()(int k, int dj, int di) const {
+    if (dj == 0 && di == 0)
+      return k == 0 ? a0 : (k == 1 ? a1 : (k == 2 ? a2 : (k == 3 ? a3 : a4)));
+    return k == 3 ? a3e : (k == 2 ? a2s : (k == 1 ? a1s : a0s));
+  }
+};
+// the row of the cell at element e of a level's five planes (PL values each,
+// row length n), every load at once
+template <typename T>
+__device__ __forceinline__ void load_row(ARow<T>& r, const T* A, uint32_t PL, uint32_t n,
+                                         uint32_t e) {
+  r.a4 = ld32(A, 4 * PL + e);
+  r.a0 = ld32(A, e);
+  r.a1 = ld32(A, PL + e);
+  r.a2 = ld32(A, 2 * PL + e);
+  r.a3 = ld32(A, 3 * PL + e);
+  r.a3e = ld32(A, 3 * PL + e + 1);
+  r.a2s = ld32(A, 2 * PL + e + n - 1);
+  r.a1s = ld32(A, PL + e + n);
+  r.a0s = ld32(A, e + n + 1);
+}
+
 }  // namespace f2d
