@@ -64,6 +64,8 @@ SIGNATURES = {
     "f2d_restrict_f64": [_p, _p, _i, _p, _i, _i, _i, _i, _p],
     "f2d_interpolate_f64": [_p, _p, _p, _i, _p, _i, _i, _i, _i, _i, _p],
     "f2d_coarsenmatrix_f64": [_p, _p, _p, _i, _p, _i, _i, _i, _i, _p],
+    "f2d_scalars_f64": [_pp],
+    "f2d_scalars_read_f64": [_p, _i],
     "f2d_norm2_f64": [_p, _p, _i, _i, _i, _p, _p],
     "f2d_kemaxu_f64": [_p, _p, _p, _i, _i, _i, _p, _p],
     "f2d_dotprod_f64": [_p, _p, _p, _i, _i, _i, _p, _p],
@@ -101,6 +103,7 @@ SIGNATURES = {
 _RESTYPE = {"f2d_last_error": C.c_char_p}
 
 _lib = None
+_fns = {}  # the library's functions by name
 
 
 def load():
@@ -134,7 +137,11 @@ def check(rc):
 
 
 def call(name, *args):
-    return check(getattr(load(), name)(*args))
+    f = _fns.get(name)
+    if f is None:
+        f = _fns[name] = getattr(load(), name)
+    rc = f(*args)
+    return check(rc) if rc else rc
 
 
 def device_count():

@@ -14,6 +14,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -867,6 +868,56 @@ static int red_scratch(double** partial) {
   static thread_local double* p = nullptr;
   if (!p) TRY(dalloc(&p, (size_t)kRedMaxBlocks * 8));
   *partial = p;
+  return F2D_OK;
+}
+
+// Results of the calling thread's reductions in pinned host memory, which
+// every device writes: one synchronization of the null stream instead of an
+// allocation, a copy and a free for each scalar (2048 x 1024, a pass of seven
+// reductions: 208 us with those, 140 so).  A thread keeps its eight values
+// until it ends, then they go to the next thread that asks.
+namespace {
+constexpr int kScalars = 8;
+std::mutex g_scalars_mu;
+std::vector<double*> g_scalars_free;
+struct ThreadScalars {
+  double* p = nullptr;
+  ~ThreadScalars() {
+    if (!p) return;
+    std::lock_guard<std::mutex> lk(g_scalars_mu);
+    try {
+      g_scalars_free.push_back(p);
+    } catch (...) {
+    }
+  }
+};
+thread_local ThreadScalars t_scalars;
+}  // namespace
+
+int f2d_scalars_f64(double** out) {
+  double*& p = t_scalars.p;
+  if (!p) {
+    std::lock_guard<std::mutex> lk(g_scalars_mu);
+    if (!g_scalars_free.empty()) {
+      p = g_scalars_free.back();
+      g_scalars_free.pop_back();
+    }
+  }
+  if (!p) {
+    void* q = nullptr;
+    const hipError_t e = hipHostMalloc(&q, kScalars * sizeof(double), hipHostMallocPortable);
+    if (e != hipSuccess) return fail(F2D_E_NOMEM, "hipHostMalloc: %s", hipGetErrorString(e));
+    p = (double*)q;
+  }
+  *out = p;
+  return F2D_OK;
+}
+
+int f2d_scalars_read_f64(double* dst, int count) {
+  const double* p = t_scalars.p;
+  if (!p || count < 0 || count > kScalars) return fail(F2D_E_ARG, "no such scalars");
+  HIPCHK(hipStreamSynchronize(nullptr));
+  std::copy(p, p + count, dst);
   return F2D_OK;
 }
 

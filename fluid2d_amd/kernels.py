@@ -38,7 +38,7 @@ import ctypes as C
 import numpy as np
 
 from . import _lib
-from .device import DeviceArray, ptr
+from .device import ptr
 
 NH = 3
 
@@ -47,9 +47,13 @@ def _shape(a):
     return a.shape[-2], a.shape[-1]
 
 
+_CST = C.c_double * 5
+
+
 def _cst(cst):
-    c = (C.c_double * 5)(*[float(v) for v in np.asarray(cst).ravel()[:5]])
-    return c
+    if type(cst) not in (list, tuple) or len(cst) < 5 or any(type(v) is not float for v in cst):
+        cst = [float(v) for v in np.asarray(cst).ravel()[:5]]
+    return _CST(*cst[:5])
 
 
 def adv_upwind(msk, x, y, u, v, cst, nh, method, order, xflx=None, yflx=None, stream=None):
@@ -120,9 +124,11 @@ def coarsenmatrix(Afine, msk1, msk2, nh, Acoarse, stream=None):
 
 
 def _scalar_call(name, nout, *args):
-    out = DeviceArray((nout,), np.float64)
-    _lib.call(name, *args, out.ptr, None)
-    return out.get()
+    buf, out = C.c_void_p(), (C.c_double * nout)()
+    _lib.call("f2d_scalars_f64", C.byref(buf))
+    _lib.call(name, *args, buf, None)
+    _lib.call("f2d_scalars_read_f64", out, nout)
+    return out
 
 
 def computenorm(msk, x, nh):

@@ -120,6 +120,12 @@ int f2d_interpolate_f64(const int8_t *msk1, const int8_t *msk2, const double *x2
 int f2d_coarsenmatrix_f64(const double *Af, const int8_t *msk1, const int8_t *msk2, int nh,
                           double *Ac, int m1, int n1, int m2, int n2, f2d_stream_t stream);
 
+/* Eight doubles of pinned host memory of the calling thread, which a reduction
+ * below takes as `out`; and, once the work on the null stream is done, the
+ * first `count` of them. */
+int f2d_scalars_f64(double **out);
+int f2d_scalars_read_f64(double *dst, int count);
+
 /* core/gmg/fortran_multigrid.f90:813-839 computenorm: out[0] = sum of x^2
  * over the fluid interior (device scalar; summation order differs from the
  * serial reference by rounding only). */
