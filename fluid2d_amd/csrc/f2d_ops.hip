@@ -965,12 +965,16 @@ template <typename T>
 void launch_mask_mul(T* x, const int8_t* mk, size_t cnt, hipStream_t s) {
   hipLaunchKernelGGL(k_mask_mul<T>, grid1(cnt), B1, 0, s, x, mk, cnt);
 }
-// Whether the two sweeps go in one pass over the operator (k_smooth2): where
-// 32-bit byte offsets reach its five planes (about 10^8 cells).  Measured
-// against two single sweeps, us: 64^2 9.6 / 9.6, 512^2 9.1 / 10.6,
-// 1024 x 512 12.0 / 17.7, 1024^2 18.8 / 29.8, 2048^2 58 / 101,
-// 4096 x 2048 152 / 228.
-static bool smooth_one_pass(int m, int n) { return 5. * 8. * m * n < 4294967296.; }
+// Whether the two sweeps go in one pass over the operator (k_smooth2): from
+// about 2 10^5 cells, below which its longer chain costs more than the bytes
+// it saves, and where 32-bit byte offsets reach the five planes (10^8 cells).
+// Kernel times, one pass (with the rims) / two single sweeps, us: 64^2 8.0 /
+// 5.4, 256^2 8.5 / 6.6, 780 x 142 8.5 / 7.3, 512^2 9.0 / 10.4; calls:
+// 1024 x 512 12.0 / 17.7, 1024^2 18.8 / 29.8, 2048^2 58 / 101, 4096 x 2048
+// 152 / 228.
+static bool smooth_one_pass(int m, int n) {
+  return (double)(m - 2 * NH) * (n - 2 * NH) >= 196608. && 5. * 8. * m * n < 4294967296.;
+}
 template <typename T>
 void launch_smooth(const int8_t* msk, const T* A, T* x, const T* b, double omega, T* t, int m,
                    int n, hipStream_t s) {

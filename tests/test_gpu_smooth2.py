@@ -1,6 +1,7 @@
-"""The one-pass double sweep of the kernel-level smoother at the edges of its
-64 x 16 tiles, on a random operator, mask and halo, against the oracle: the
-same bits (same operations in the same order)."""
+"""The double sweep of the kernel-level smoother, in one pass (from 196608
+cells) at the edges of its 64 x 16 tiles and in two below, on a random
+operator, mask and halo, against the oracle: the same bits (same operations in
+the same order)."""
 import numpy as np
 import pytest
 
@@ -12,7 +13,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("ny,nx", [(4, 4), (15, 63), (16, 64), (17, 65), (18, 66), (34, 130),
-                                   (5, 200), (97, 6), (256, 192)])
+                                   (5, 200), (97, 6), (256, 192), (448, 448),
+                                   (449, 449), (447, 511), (466, 450), (4, 50001), (33000, 6)])
 def test_double_sweep_at_tile_edges(ny, nx):
     rng = np.random.default_rng(100 * ny + nx)
     m, n = ny + 2 * NH, nx + 2 * NH
