@@ -183,11 +183,13 @@ struct TrVal {
 // of stage state and tendencies), 1024^2 one tracer 20.9 -> 17.1 us (the last
 // stage 5 TB/s), 128^2 12.2 -> 7.1 us, 32 mixed instances of 64^2..512^2 49.1
 // -> 36.4 us.
+// Launch bounds: two FP64 tracers in 128 registers, not 130, so that a compute
+// unit holds four workgroups and 2048 x 1024 runs in two rounds (46.9 -> 42.7
+// us); the FP32 form would spill (384 x 192 steps 361 -> 363 us).
 template <typename T, int NTR, bool UP>
-__global__ void __launch_bounds__(256) k_rhs(const Task* __restrict__ tasks,
-                                             const InstD* __restrict__ I, double* P, T* Q,
-                                             const int8_t* __restrict__ B,
-                                             const DynD* __restrict__ dyn, int stage, int out_k) {
+__global__ void __launch_bounds__(256, NTR == 2 && sizeof(T) == 8 ? 4 : 1)
+    k_rhs(const Task* __restrict__ tasks, const InstD* __restrict__ I, double* P, T* Q,
+          const int8_t* __restrict__ B, const DynD* __restrict__ dyn, int stage, int out_k) {
   constexpr int RS = 4;  // rows of a strip
   static_assert(TY == 4 * RS && TX == 64, "one wavefront per strip row");
   __shared__ double qs[NTR][QH * QW];
