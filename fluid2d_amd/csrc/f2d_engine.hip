@@ -27,6 +27,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <memory>
 #include <functional>
 #include <string>
 #include <type_traits>
@@ -4548,6 +4549,9 @@ static int merge_persistent(Batch& b, std::vector<Launch>& prog) {
 static int upload_programs(Batch& b);
 static int build_programs(Batch& b) {
   b.tasks.clear();
+  // address space for the lists, so that they do not move as they grow (32
+  // instances hold 5.7 10^5 tasks); pages never written cost nothing
+  b.tasks.reserve(std::min((size_t)b.ninst << 15, (size_t)1 << 21));
   b.spans.clear();
   b.slots.clear();
   b.prog_init.clear();
@@ -4647,9 +4651,9 @@ static int upload_programs(Batch& b) {
   // kernel's workgroup k takes task k, its instance first + k), each task's
   // slot its index in the builder's list.  Persistent phases keep the
   // builder's order (the persistent kernel walks them itself).
-  std::vector<Task> dev(b.tasks);
-  for (size_t k = 0; k < dev.size(); k++) dev[k].slot = 0;
-  std::vector<char> placed(b.tasks.size(), 0);
+  const size_t ntask = b.tasks.size();
+  std::unique_ptr<Task[]> dev(new Task[ntask]);  // each entry is written below
+  std::vector<char> placed(ntask, 0);
   for (auto* pr : progs)
     for (Launch& L : *pr) {
       if (L.ntask <= 0 || L.kind == L_FOLD || L.kind == L_GATE || L.kind == L_PERSIST) continue;
@@ -4666,7 +4670,12 @@ static int upload_programs(Batch& b) {
         placed[L.toff + k] = 1;
       }
     }
-  ECHK(hipMemcpy(b.dT, dev.data(), dev.size() * sizeof(Task), hipMemcpyHostToDevice));
+  for (size_t k = 0; k < ntask; k++)
+    if (!placed[k]) {
+      dev[k] = b.tasks[k];
+      dev[k].slot = 0;
+    }
+  ECHK(hipMemcpy(b.dT, dev.get(), ntask * sizeof(Task), hipMemcpyHostToDevice));
   if (b.dPh) (void)hipFree(b.dPh);
   if (b.bar) (void)hipFree(b.bar);
   b.dPh = nullptr;
@@ -5135,13 +5144,16 @@ int f2d_batch_create(int ninst, const f2d_model_params* params, const int8_t* co
         return bail(efail(F2D_E_ARG, "level shape mismatch"));
       }
       bool ok = true;
-      if (b->prec == 0) {
-        ok = hipMemcpy((double*)b->Q + d.L[l].A, gA, 5 * S * sizeof(double),
-                       hipMemcpyDeviceToDevice) == hipSuccess;
-      } else {  // operators rounded to FP32 for the FP32 V-cycles
-        std::vector<double> hA(5 * S);
-        std::vector<float> fA(5 * S);
+      std::vector<double> hA;  // the operator on the host, copied where it is needed
+      if (b->prec != 0 || l == 0 || S <= COARSE_CELLS) {
+        hA.resize(5 * S);
         ok = hipMemcpy(hA.data(), gA, 5 * S * sizeof(double), hipMemcpyDeviceToHost) == hipSuccess;
+      }
+      if (b->prec == 0) {
+        ok = ok && hipMemcpy((double*)b->Q + d.L[l].A, gA, 5 * S * sizeof(double),
+                             hipMemcpyDeviceToDevice) == hipSuccess;
+      } else {  // operators rounded to FP32 for the FP32 V-cycles
+        std::vector<float> fA(5 * S);
         for (size_t q = 0; q < 5 * S; q++) fA[q] = (float)hA[q];
         ok = ok && hipMemcpy((float*)b->Q + d.L[l].A, fA.data(), 5 * S * sizeof(float),
                              hipMemcpyHostToDevice) == hipSuccess;
@@ -5150,9 +5162,6 @@ int f2d_batch_create(int ninst, const f2d_model_params* params, const int8_t* co
         ok = ok && hipMemcpy(b->P + d.A0d, gA, 5 * S * sizeof(double),
                              hipMemcpyDeviceToDevice) == hipSuccess;
         // stencil bits of the finest operator, verified value by value
-        std::vector<double> hA(5 * S);
-        ok = ok && hipMemcpy(hA.data(), gA, 5 * S * sizeof(double), hipMemcpyDeviceToHost) ==
-                       hipSuccess;
         // bits 0-3: coupling A_k nonzero (all nonzero values of a plane
         // equal); bit 4: the cell mask.  The centre coefficient is read
         // only where the mask is set (Jacobi and residual are 0 elsewhere),
@@ -5189,11 +5198,9 @@ int f2d_batch_create(int ninst, const f2d_model_params* params, const int8_t* co
       if (l > 0 && S <= COARSE_CELLS) {  // host copies for the packed coarse operands
         std::vector<double>& cA = h.cA[l];
         std::vector<int8_t>& cM = h.cM[l];
-        cA.resize(5 * S);
+        cA.swap(hA);
         cM.resize(S);
-        ok = ok &&
-             hipMemcpy(cA.data(), gA, 5 * S * sizeof(double), hipMemcpyDeviceToHost) == hipSuccess &&
-             hipMemcpy(cM.data(), gm, S, hipMemcpyDeviceToHost) == hipSuccess;
+        ok = ok && hipMemcpy(cM.data(), gm, S, hipMemcpyDeviceToHost) == hipSuccess;
         if (b->prec != 0)  // the pool's rounding
           for (double& a : cA) a = (double)(float)a;
       }
