@@ -546,7 +546,10 @@ __device__ __forceinline__ void store_img_mask(PA a, const int8_t* mk, int J, in
   if (jm && im) put(J - M, I - N);
 }
 
-// store_img_mask with 32-bit offsets (see ld32)
+// store_img_mask with 32-bit offsets (see ld32).  A cell has at most one image
+// per axis where both have at least 2 NH interior cells (uniform over the
+// tile): three stores then, not eight tests (1024^2 steps 1502 -> 1465
+// us, whose wall tiles spent 4.6 us on the second sweep and its stores).
 template <typename T>
 __device__ __forceinline__ void store_img_mask32(T* a, const int8_t* mk, int J, int I, T v, int m,
                                                  int n) {
@@ -555,8 +558,17 @@ __device__ __forceinline__ void store_img_mask32(T* a, const int8_t* mk, int J, 
     st32(a, c, mk ? v * T(ld32(mk, c)) : v);
   };
   put(J, I);
-  if (J >= 2 * NH && J < m - 2 * NH && I >= 2 * NH && I < n - 2 * NH) return;  // no image
+  const bool jl = J < 2 * NH, jh = J >= m - 2 * NH, il = I < 2 * NH, ih = I >= n - 2 * NH;
+  const bool jo = jl || jh, io = il || ih;
+  if (!jo && !io) return;  // no image
   const int M = m - 2 * NH, N = n - 2 * NH;
+  if (M >= 2 * NH && N >= 2 * NH) {
+    const int j = jl ? J + M : J - M, i = il ? I + N : I - N;
+    if (jo) put(j, I);
+    if (io) put(J, i);
+    if (jo && io) put(j, i);
+    return;
+  }
   const bool jp = J + M < m && J + M >= m - NH, jm = J - M >= 0 && J - M < NH;
   const bool ip = I + N < n && I + N >= n - NH, im = I - N >= 0 && I - N < NH;
   if (jp) put(J + M, I);
