@@ -137,10 +137,11 @@ def check(rc):
 
 
 def call(name, *args):
-    f = _fns.get(name)
-    if f is None:
-        f = _fns[name] = getattr(load(), name)
-    rc = f(*args)
+    try:
+        rc = _fns[name](*args)
+    except KeyError:
+        _fns[name] = getattr(load(), name)
+        rc = _fns[name](*args)
     return check(rc) if rc else rc
 
 

@@ -81,6 +81,5 @@ def ptr(a):
         return None
     if isinstance(a, DeviceArray):
         return a.ptr
-    if hasattr(a, "data_ptr"):
-        return a.data_ptr()
-    return int(a)
+    f = getattr(a, "data_ptr", None)
+    return f() if f is not None else int(a)

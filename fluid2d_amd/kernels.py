@@ -44,7 +44,8 @@ NH = 3
 
 
 def _shape(a):
-    return a.shape[-2], a.shape[-1]
+    s = a.shape
+    return s[-2], s[-1]
 
 
 _CST = C.c_double * 5
