@@ -472,9 +472,9 @@ __global__ void __launch_bounds__(256) k_c2c(const Task* __restrict__ tasks,
 // beyond that.  Launch bounds that fit one more workgroup spill and lose
 // (2048 x 1024 in 8-row tiles at 64 registers 23.1 us, at 74 17.5).
 // With threads on every fourth row, the right-hand side in LDS and the
-// operator read by each sweep: 1024^2 12.5 us, now 10.6; 2048 x 1024 18.4,
-// now 17.5; explicit 1024 x 512 13.2, now 11.8; whole steps of 1024^2 1535,
-// now 1497 us.
+// operator read by each sweep: 1024^2 12.5 us, now 10.0; 2048 x 1024 18.4,
+// now 17.2; explicit 1024 x 512 13.2, now 11.7; whole steps of 1024^2 1535,
+// then 1497 us.
 // Phase timestamps of the 64 x 16 smoother tiles (profiling build only,
 // make stamps): thread 0 of each of the first 2048 workgroups of a launch
 // records the real-time clock (100 MHz) at the start, after the tile loads

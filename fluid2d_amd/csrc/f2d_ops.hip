@@ -4,7 +4,7 @@
 // One work-item per output cell; workgroups of 64 x 4 (one wavefront per
 // row segment, so every load and store of a row is a coalesced 512-byte
 // sweep in FP64).  These are the building blocks; the fused/LDS-tiled
-// variants live in f2d_fused.hip.  Each kernel cites the reference routine
+// variants live in f2d_engine.hip.  Each kernel cites the reference routine
 // whose arithmetic (operation order included) it reproduces.
 #include <algorithm>
 #include <type_traits>

@@ -52,9 +52,12 @@ _CST = C.c_double * 5
 
 
 def _cst(cst):
-    if type(cst) not in (list, tuple) or len(cst) < 5 or any(type(v) is not float for v in cst):
-        cst = [float(v) for v in np.asarray(cst).ravel()[:5]]
-    return _CST(*cst[:5])
+    if type(cst) in (list, tuple):
+        try:  # flat numbers
+            return _CST(*cst[:5])
+        except TypeError:
+            pass
+    return _CST(*[float(v) for v in np.asarray(cst).ravel()[:5]])
 
 
 def adv_upwind(msk, x, y, u, v, cst, nh, method, order, xflx=None, yflx=None, stream=None):
