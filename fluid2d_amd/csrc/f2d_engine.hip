@@ -4935,8 +4935,17 @@ static int hierarchy_build(Hierarchy& H, int nlev, const HierLevel* L, const uin
 int hierarchy_create(int nlev, const HierLevel* L, const uint8_t* bits, const double* w0,
                      double omega, Hierarchy** out) {
   *out = nullptr;
-  // what the fused kernels take: at least two levels, arrays below 4 GiB
+  // what the fused kernels take: at least two levels, arrays below 4 GiB, and
+  // a coarsest level whose operands fit the coarse kernel's LDS (thin grids
+  // end at up to a quarter of their long side: 256 x 4 under 1024 x 16)
   if (nlev < 2 || nlev > MAXLEV || (double)L[0].m * L[0].n * 40. >= 4294967296.) return F2D_OK;
+  {
+    InstD d;
+    d.nlev = nlev;
+    d.L[nlev - 1].m = L[nlev - 1].m;
+    d.L[nlev - 1].n = L[nlev - 1].n;
+    if (coarse_bytes(d, nlev - 1, sizeof(double)) > lds_budget(0)) return F2D_OK;
+  }
   Hierarchy* H = new Hierarchy();
   const int rc = hierarchy_build(*H, nlev, L, bits, w0, omega);
   if (rc) {
