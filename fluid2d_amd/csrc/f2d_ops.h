@@ -19,6 +19,9 @@ struct Scale8 {
 struct St9 {
   double w[9];
 };
+struct W5 {
+  double v[5];
+};
 
 template <typename T>
 void launch_adv_upwind(const int8_t* msk, const T* x, T* y, const T* u, const T* v, T* xflx,
@@ -83,8 +86,9 @@ void launch_coarsen(const double* Af, const int8_t* msk1, const int8_t* msk2, do
                     int n1, int m2, int n2, hipStream_t s);
 void launch_afinest(const int8_t* msk, double* A, const St9& st, double coef, int m, int n,
                     hipStream_t s);
+// (bad[0] = 1 where bits and weights are not the operator; else untouched)
 void launch_stencil_bits(const int8_t* msk, const double* A, uint8_t* bits, int m, int n,
-                         hipStream_t s);
+                         const W5& w, double* bad, hipStream_t s);
 void launch_corner_mask(const int8_t* msk, int8_t* mskp, int m, int n, hipStream_t s);
 // A5 -= shift wherever A5 != 0 (the Helmholtz operator of core/gmg/hierarchy.py:80-84)
 void launch_helmholtz_shift(double* A5, size_t cnt, double shift, hipStream_t s);

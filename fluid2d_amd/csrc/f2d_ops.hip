@@ -531,14 +531,23 @@ __global__ void k_afinest(const int8_t* __restrict__ msk, double* __restrict__ A
 }
 
 // Stencil bits of the level-0 operator (five planes): bit k (k < 4) where
-// coupling A_k is nonzero, bit 4 the cell mask.
+// coupling A_k is nonzero, bit 4 the cell mask.  bad[0] = 1 where the bits and
+// the weights w do not give the operator back: a coupling that is neither 0
+// nor its weight, or the centre of a cell with a mask (read nowhere else)
+// that is not its weight.
 __global__ void k_stencil_bits(const int8_t* __restrict__ msk, const double* __restrict__ A,
-                               uint8_t* __restrict__ bits, size_t cnt) {
+                               uint8_t* __restrict__ bits, size_t cnt, W5 w, double* bad) {
   const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= cnt) return;
   unsigned b = msk[q] != 0 ? 16u : 0u;
-  for (int k = 0; k < 4; k++) b |= A[k * cnt + q] != 0. ? 1u << k : 0u;
+  bool ok = b == 0u || A[4 * cnt + q] == w.v[4];
+  for (int k = 0; k < 4; k++) {
+    const double a = A[k * cnt + q];
+    ok = ok && (a == 0. || a == w.v[k]);
+    b |= a != 0. ? 1u << k : 0u;
+  }
   bits[q] = (uint8_t)b;
+  if (!ok) bad[0] = 1.;
 }
 
 // Corner mask (core/operators.py:59-67): 1 where celltocorner(msk) == 1.
@@ -1087,9 +1096,9 @@ void launch_helmholtz_shift(double* A5, size_t cnt, double shift, hipStream_t s)
   hipLaunchKernelGGL(k_helmholtz_shift, grid1(cnt), B1, 0, s, A5, cnt, shift);
 }
 void launch_stencil_bits(const int8_t* msk, const double* A, uint8_t* bits, int m, int n,
-                         hipStream_t s) {
+                         const W5& w, double* bad, hipStream_t s) {
   const size_t cnt = (size_t)m * n;
-  hipLaunchKernelGGL(k_stencil_bits, grid1(cnt), B1, 0, s, msk, A, bits, cnt);
+  hipLaunchKernelGGL(k_stencil_bits, grid1(cnt), B1, 0, s, msk, A, bits, cnt, w, bad);
 }
 void launch_corner_mask(const int8_t* msk, int8_t* mskp, int m, int n, hipStream_t s) {
   hipLaunchKernelGGL(k_corner_mask, grid2(n, m), B2, 0, s, msk, mskp, m, n);

@@ -102,8 +102,8 @@ struct f2d_gmg {
   double* scal = nullptr;     // device scalars
   double* hscal = nullptr;    // pinned host mirror
   hipStream_t s = nullptr;
-  double w0[5] = {0., 0., 0., 0., 0.};  // level-0 operator: weights, and its
-  uint8_t* bits = nullptr;              // stencil bits
+  W5 w0 = {{0., 0., 0., 0., 0.}};  // level-0 operator: weights, and its
+  uint8_t* bits = nullptr;         // stencil bits
   // the cycles of solve and twoVcycle on the engine's fused kernels; null:
   // one launch per routine
   eng::Hierarchy* fused = nullptr;
@@ -210,7 +210,7 @@ static int gmg_build(int nx, int ny, double dx, double dy, double hydroepsilon, 
       memcpy(st.w, w, sizeof w);
     }
     launch_afinest(L.msk, A9[0], st, 1. / (dx * dy), L.m, L.n, s);
-    for (int k = 0; k < 5; k++) g->w0[k] = st.w[k] * (1. / (dx * dy)) * 1. * 1.;
+    for (int k = 0; k < 5; k++) g->w0.v[k] = st.w[k] * (1. / (dx * dy)) * 1. * 1.;
   }
   for (int l = 1; l < g->nlev; l++) {
     Level &F = g->L[l - 1], &C = g->L[l];
@@ -231,23 +231,28 @@ static int gmg_build(int nx, int ny, double dx, double dy, double hydroepsilon, 
   return F2D_OK;
 }
 
-// (Re)builds the fused cycles of a hierarchy from its operators.  Every
-// value of a level-0 plane is its weight or 0 by construction (launch_afinest;
-// the Helmholtz shift changes every nonzero centre alike).
+// (Re)builds the fused cycles of a hierarchy from its operators, which take
+// the level-0 operator as stencil bits and weights.  Every value of a plane is
+// its weight or 0 on masks of 0 and 1 (the Helmholtz shift changes every
+// nonzero centre alike); an operator that is anything else keeps one launch
+// per routine.
 static int gmg_fuse(f2d_gmg* g) {
   eng::hierarchy_destroy(g->fused);
   g->fused = nullptr;
   const Level& L0 = g->L[0];
   if (!g->bits) TRY(dalloc(&g->bits, L0.size()));
-  launch_stencil_bits(L0.msk, L0.A, g->bits, L0.m, L0.n, g->s);
+  launch_fill_value(g->scal, 0., 1, g->s);
+  launch_stencil_bits(L0.msk, L0.A, g->bits, L0.m, L0.n, g->w0, g->scal, g->s);
   LAUNCHCHK();
+  HIPCHK(hipMemcpyAsync(g->hscal, g->scal, 8, hipMemcpyDeviceToHost, g->s));
   HIPCHK(hipStreamSynchronize(g->s));
+  if (g->hscal[0] != 0.) return F2D_OK;
   std::vector<eng::HierLevel> v(g->nlev);
   for (int l = 0; l < g->nlev; l++) {
     const Level& L = g->L[l];
     v[l] = eng::HierLevel{L.m, L.n, L.msk, L.A, L.x, L.b, L.t};
   }
-  const int rc = eng::hierarchy_create(g->nlev, v.data(), g->bits, g->w0, g->omega, &g->fused);
+  const int rc = eng::hierarchy_create(g->nlev, v.data(), g->bits, g->w0.v, g->omega, &g->fused);
   return rc ? fail(rc, "%s", eng::hierarchy_error()) : F2D_OK;
 }
 
@@ -1052,7 +1057,7 @@ int f2d_gmg_set_helmholtz(f2d_gmg* g, double Rd) {
     launch_helmholtz_shift(g->L[l].A + 4 * g->L[l].size(), g->L[l].size(), shift, g->s);
   LAUNCHCHK();
   HIPCHK(hipStreamSynchronize(g->s));
-  g->w0[4] -= shift;
+  g->w0.v[4] -= shift;
   return gmg_fuse(g);
 }
 int f2d_gmg_nlevels(const f2d_gmg* g, int* nlev) {
