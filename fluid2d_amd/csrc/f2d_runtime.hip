@@ -107,6 +107,12 @@ struct f2d_gmg {
   // the cycles of solve and twoVcycle on the engine's fused kernels; null:
   // one launch per routine
   eng::Hierarchy* fused = nullptr;
+  // A level array that the fused cycles hold a copy of (operator, mask) or do
+  // not keep (r, and x and b below the finest level) has been handed out: the
+  // caller may write the one and read the other, so from then on the cycles
+  // run one launch per routine, on the arrays themselves.
+  mutable bool shown = false;
+  bool use_fused() const { return fused && !shown; }
 };
 
 static int gmg_free(f2d_gmg* g) {
@@ -332,7 +338,7 @@ static int g_solve(f2d_gmg* g, double* x, const double* b, int maxite, double to
   double res0 = nb0 / normeb, res = res0;
   int nite = 0, ndiv = 0;
   while (nite < maxite && res0 > tol) {
-    if (g->fused) {
+    if (g->use_fused()) {
       const int rc = eng::hierarchy_run(g->fused, 1, g->s);
       if (rc) return fail(rc, "%s", eng::hierarchy_error());
     } else {
@@ -364,7 +370,7 @@ static int g_twovcycle(f2d_gmg* g, double* x, const double* b) {
   Level& L0 = g->L[0];
   launch_copy(L0.x, (const double*)x, L0.size(), g->s);
   launch_copy(L0.b, b, L0.size(), g->s);
-  if (g->fused) {
+  if (g->use_fused()) {
     const int rc = eng::hierarchy_run(g->fused, 0, g->s);
     if (rc) return fail(rc, "%s", eng::hierarchy_error());
   } else {
@@ -1076,6 +1082,7 @@ int f2d_gmg_level(const f2d_gmg* g, int lev, int which, void** dev_ptr, int* m, 
     case 4: p = L.r; break;
     default: return fail(F2D_E_ARG, "which must be 0..4");
   }
+  if (which <= 1 || which == 4 || lev > 0) g->shown = true;
   *dev_ptr = p;
   *m = L.m;
   *n = L.n;

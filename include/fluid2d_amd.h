@@ -185,7 +185,10 @@ int f2d_gmg_destroy(f2d_gmg *g);
  * after f2d_gmg_create and before any cycle. */
 int f2d_gmg_set_helmholtz(f2d_gmg *g, double Rd);
 int f2d_gmg_nlevels(const f2d_gmg *g, int *nlev);
-/* which: 0 msk (int8), 1 A (5 planes), 2 x, 3 b, 4 r */
+/* which: 0 msk (int8), 1 A (5 planes), 2 x, 3 b, 4 r.  The array itself, also
+ * to write to.  Any but x and b of level 0 moves f2d_gmg_solve and
+ * f2d_gmg_twovcycle from fused kernels, which hold copies of A and msk and do
+ * not keep the others, to one kernel per routine on the arrays, for good. */
 int f2d_gmg_level(const f2d_gmg *g, int lev, int which, void **dev_ptr, int *m, int *n);
 /* core/gmg/hierarchy.py:98-126 Vcycle(lev1), :131-151 Fcycle(lev1) */
 int f2d_gmg_vcycle(f2d_gmg *g, int lev1);
