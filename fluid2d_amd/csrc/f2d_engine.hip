@@ -4947,7 +4947,12 @@ int hierarchy_create(int nlev, const HierLevel* L, const uint8_t* bits, const do
     if (coarse_bytes(d, nlev - 1, sizeof(double)) > lds_budget(0)) return F2D_OK;
   }
   Hierarchy* H = new Hierarchy();
-  const int rc = hierarchy_build(*H, nlev, L, bits, w0, omega);
+  int rc;
+  try {
+    rc = hierarchy_build(*H, nlev, L, bits, w0, omega);
+  } catch (const std::bad_alloc&) {
+    rc = efail(F2D_E_NOMEM, "host memory of the launch programs");
+  }
   if (rc) {
     hierarchy_free(H);
     return rc;

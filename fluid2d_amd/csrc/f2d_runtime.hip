@@ -104,15 +104,16 @@ struct f2d_gmg {
   hipStream_t s = nullptr;
   W5 w0 = {{0., 0., 0., 0., 0.}};  // level-0 operator: weights, and its
   uint8_t* bits = nullptr;         // stencil bits
-  // the cycles of solve and twoVcycle on the engine's fused kernels; null:
-  // one launch per routine
+  // the cycles of solve and twoVcycle on the engine's fused kernels, built by
+  // the first call that runs them (gmg_fused); null once tried: one launch per
+  // routine
   eng::Hierarchy* fused = nullptr;
+  bool tried = false;
   // A level array that the fused cycles hold a copy of (operator, mask) or do
   // not keep (r, and x and b below the finest level) has been handed out: the
   // caller may write the one and read the other, so from then on the cycles
   // run one launch per routine, on the arrays themselves.
   mutable bool shown = false;
-  bool use_fused() const { return fused && !shown; }
 };
 
 static int gmg_free(f2d_gmg* g) {
@@ -237,14 +238,12 @@ static int gmg_build(int nx, int ny, double dx, double dy, double hydroepsilon, 
   return F2D_OK;
 }
 
-// (Re)builds the fused cycles of a hierarchy from its operators, which take
-// the level-0 operator as stencil bits and weights.  Every value of a plane is
-// its weight or 0 on masks of 0 and 1 (the Helmholtz shift changes every
-// nonzero centre alike); an operator that is anything else keeps one launch
-// per routine.
+// Builds the fused cycles of a hierarchy from its operators, which take the
+// level-0 operator as stencil bits and weights.  Every value of a plane is its
+// weight or 0 on masks of 0 and 1 (the Helmholtz shift changes every nonzero
+// centre alike); an operator that is anything else keeps one launch per
+// routine.
 static int gmg_fuse(f2d_gmg* g) {
-  eng::hierarchy_destroy(g->fused);
-  g->fused = nullptr;
   const Level& L0 = g->L[0];
   if (!g->bits) TRY(dalloc(&g->bits, L0.size()));
   launch_fill_value(g->scal, 0., 1, g->s);
@@ -260,6 +259,19 @@ static int gmg_fuse(f2d_gmg* g) {
   }
   const int rc = eng::hierarchy_create(g->nlev, v.data(), g->bits, g->w0.v, g->omega, &g->fused);
   return rc ? fail(rc, "%s", eng::hierarchy_error()) : F2D_OK;
+}
+
+// The fused cycles a solve or twoVcycle runs; null: one launch per routine.
+// Built here, not with the hierarchy, whose other users (Vcycle, Fcycle, the
+// arrays) would pay for them: f2d_gmg_create of 4096^2 took 56 ms with them,
+// 16 without.  Where they cannot be built (memory), the routines serve.
+static eng::Hierarchy* gmg_fused(f2d_gmg* g) {
+  if (g->shown) return nullptr;
+  if (!g->tried) {
+    g->tried = true;
+    if (gmg_fuse(g) != F2D_OK) (void)hipGetLastError();  // (not a launch's error)
+  }
+  return g->fused;
 }
 
 // core/gmg/level.py:340-368 (smooth nite times, fill after each)
@@ -337,9 +349,10 @@ static int g_solve(f2d_gmg* g, double* x, const double* b, int maxite, double to
   TRY(g_norm(g, 0, L0.b, &nb0));
   double res0 = nb0 / normeb, res = res0;
   int nite = 0, ndiv = 0;
+  eng::Hierarchy* fused = nite < maxite && res0 > tol ? gmg_fused(g) : nullptr;
   while (nite < maxite && res0 > tol) {
-    if (g->use_fused()) {
-      const int rc = eng::hierarchy_run(g->fused, 1, g->s);
+    if (fused) {
+      const int rc = eng::hierarchy_run(fused, 1, g->s);
       if (rc) return fail(rc, "%s", eng::hierarchy_error());
     } else {
       g_fcycle(g, 0);
@@ -370,8 +383,8 @@ static int g_twovcycle(f2d_gmg* g, double* x, const double* b) {
   Level& L0 = g->L[0];
   launch_copy(L0.x, (const double*)x, L0.size(), g->s);
   launch_copy(L0.b, b, L0.size(), g->s);
-  if (g->use_fused()) {
-    const int rc = eng::hierarchy_run(g->fused, 0, g->s);
+  if (eng::Hierarchy* fused = gmg_fused(g)) {
+    const int rc = eng::hierarchy_run(fused, 0, g->s);
     if (rc) return fail(rc, "%s", eng::hierarchy_error());
   } else {
     for (int k = 0; k < 2; k++) g_vcycle(g, 0);
@@ -1047,13 +1060,7 @@ int f2d_domain_sum_f64_noalloc(const double* x, int nh, int m, int n, double* ou
 int f2d_gmg_create(int nx, int ny, int nh, double dx, double dy, double hydroepsilon, double omega,
                    const int8_t* mskp_host, f2d_gmg** out) {
   if (nh != NH) return fail(F2D_E_ARG, "nh must be 3");
-  TRY(gmg_build(nx, ny, dx, dy, hydroepsilon, omega, mskp_host, out));
-  const int rc = gmg_fuse(*out);
-  if (rc) {
-    gmg_free(*out);
-    *out = nullptr;
-  }
-  return rc;
+  return gmg_build(nx, ny, dx, dy, hydroepsilon, omega, mskp_host, out);
 }
 int f2d_gmg_destroy(f2d_gmg* g) { return gmg_free(g); }
 int f2d_gmg_set_helmholtz(f2d_gmg* g, double Rd) {
@@ -1064,7 +1071,10 @@ int f2d_gmg_set_helmholtz(f2d_gmg* g, double Rd) {
   LAUNCHCHK();
   HIPCHK(hipStreamSynchronize(g->s));
   g->w0.v[4] -= shift;
-  return gmg_fuse(g);
+  eng::hierarchy_destroy(g->fused);
+  g->fused = nullptr;
+  g->tried = false;
+  return F2D_OK;
 }
 int f2d_gmg_nlevels(const f2d_gmg* g, int* nlev) {
   *nlev = g->nlev;
@@ -1168,8 +1178,7 @@ int f2d_model_create(const f2d_model_params* p, const int8_t* msk_host, f2d_mode
   if (hipMemcpy(mskp.data(), M->mskp, M->fsz, hipMemcpyDeviceToHost) != hipSuccess)
     return bail(fail(F2D_E_HIP, "download corner mask"));
   if ((rc = gmg_build(p->nx, p->ny, M->dx, M->dy, p->hydroepsilon, 8. / 9., mskp.data(),
-                      &M->gmg)) ||
-      (rc = gmg_fuse(M->gmg)))
+                      &M->gmg)))
     return bail(rc);
   M->cst[0] = M->dx;
   M->cst[1] = M->dy;
