@@ -105,10 +105,10 @@ struct f2d_gmg {
   W5 w0 = {{0., 0., 0., 0., 0.}};  // level-0 operator: weights, and its
   uint8_t* bits = nullptr;         // stencil bits
   // the cycles of solve and twoVcycle on the engine's fused kernels, built by
-  // the first call that runs them (gmg_fused); null once tried: one launch per
-  // routine
+  // one of the first calls (gmg_fused); null once tried: one launch per routine
   eng::Hierarchy* fused = nullptr;
   bool tried = false;
+  bool used = false;  // a solve or twoVcycle has been called
   // A level array that the fused cycles hold a copy of (operator, mask) or do
   // not keep (r, and x and b below the finest level) has been handed out: the
   // caller may write the one and read the other, so from then on the cycles
@@ -264,13 +264,20 @@ static int gmg_fuse(f2d_gmg* g) {
 // The fused cycles a solve or twoVcycle runs; null: one launch per routine.
 // Built here, not with the hierarchy, whose other users (Vcycle, Fcycle, the
 // arrays) would pay for them: f2d_gmg_create of 4096^2 took 56 ms with them,
-// 16 without.  Where they cannot be built (memory), the routines serve.
-static eng::Hierarchy* gmg_fused(f2d_gmg* g) {
+// 16 without.  A handle's first call builds them only where that one call is
+// faster for it: a solve of up to 2^22 cells (first call by routine / with the
+// build, ms: 64^2 3.6 / 0.9, 512^2 7.4 / 1.7, 2048^2 12.2 / 6.1, but 4096 x
+// 2048 14.9 / 18.4; twoVcycle 64^2 0.40 / 0.42, 512^2 0.52 / 0.90, 2048^2 1.3
+// / 4.0).  Where they cannot be built (memory), the routines serve.
+static eng::Hierarchy* gmg_fused(f2d_gmg* g, bool solve) {
   if (g->shown) return nullptr;
-  if (!g->tried) {
+  const Level& L = g->L[0];
+  const bool now = solve && (size_t)(L.m - 2 * NH) * (L.n - 2 * NH) <= (size_t)1 << 22;
+  if (!g->tried && (now || g->used)) {
     g->tried = true;
     if (gmg_fuse(g) != F2D_OK) (void)hipGetLastError();  // (not a launch's error)
   }
+  g->used = true;
   return g->fused;
 }
 
@@ -349,7 +356,7 @@ static int g_solve(f2d_gmg* g, double* x, const double* b, int maxite, double to
   TRY(g_norm(g, 0, L0.b, &nb0));
   double res0 = nb0 / normeb, res = res0;
   int nite = 0, ndiv = 0;
-  eng::Hierarchy* fused = nite < maxite && res0 > tol ? gmg_fused(g) : nullptr;
+  eng::Hierarchy* fused = nite < maxite && res0 > tol ? gmg_fused(g, true) : nullptr;
   while (nite < maxite && res0 > tol) {
     if (fused) {
       const int rc = eng::hierarchy_run(fused, 1, g->s);
@@ -383,7 +390,7 @@ static int g_twovcycle(f2d_gmg* g, double* x, const double* b) {
   Level& L0 = g->L[0];
   launch_copy(L0.x, (const double*)x, L0.size(), g->s);
   launch_copy(L0.b, b, L0.size(), g->s);
-  if (eng::Hierarchy* fused = gmg_fused(g)) {
+  if (eng::Hierarchy* fused = gmg_fused(g, false)) {
     const int rc = eng::hierarchy_run(fused, 0, g->s);
     if (rc) return fail(rc, "%s", eng::hierarchy_error());
   } else {

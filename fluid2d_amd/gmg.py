@@ -9,7 +9,9 @@ scratch (``Vcycle`` and ``Fcycle`` leave each level's x and b in them).
 fused kernels (512^2 solve 0.66 ms, by routine 4.3) until an array is handed out that
 these hold a copy of or do not keep: A, msk, r, and x and b below the finest
 level.  From then on they run one kernel per routine, with the A and msk that
-the arrays hold at the call, and leave every level's values in them.
+the arrays hold at the call, and leave every level's values in them.  The
+first solve or the second twoVcycle of a Gmg (the second solve past 2^22
+cells) sets the fused kernels up.
 """
 import ctypes as C
 
