@@ -3756,13 +3756,15 @@ struct Builder {
   }
 
   // the two programs of a stand-alone hierarchy (Gmg): two V-cycles from
-  // level 0 on its x (hierarchy.py:207-218), and an F-cycle of its b
-  void hierarchy_programs() {
+  // level 0 on its x (hierarchy.py:207-218), and an F-cycle of its b.  Both
+  // have to start from and end in x, the first of the level's two buffers.
+  int hierarchy_programs() {
     HostInst& h = b.H[0];
     const std::vector<int> who{0}, st{0};
     prog = &b.prog_step;
     vcycle(who, st, 0, 0, false);
     vcycle(who, st, 0, 0, false);
+    bool in_x = h.cur[0] == 0;
     prog = &b.prog_init;
     std::vector<Task> rs;
     rr_tasks(0, 0, 0, -1, -1, rs, pick_ty0(who) / 2);
@@ -3772,7 +3774,8 @@ struct Builder {
     fcycle_down(who, 0);
     coarse(who, 1, 0);
     fcycle_up(who, 0);
-    if (h.cur[0] != 0) fprintf(stderr, "engine: hierarchy program parity\n");
+    in_x = in_x && h.cur[0] == 0;
+    return in_x ? F2D_OK : efail(F2D_E_UNSUPPORTED, "hierarchy programs: result not in x");
   }
 
   // Defect-correction solve, core/gmg/hierarchy.py:154-192 (solve): the
@@ -4577,7 +4580,7 @@ static int build_programs(Batch& b) {
   bd.lo = 0;
   bd.hi = b.ninst;
   if (b.hierarchy) {
-    bd.hierarchy_programs();
+    ETRY(bd.hierarchy_programs());
     return upload_programs(b);
   }
   bd.prog = &b.prog_init;
