@@ -4984,10 +4984,16 @@ int hierarchy_run(Hierarchy* h, int which, hipStream_t s) {
   if (!h->exec[which]) {  // captured by the first call that needs it
     ECHK(hipStreamBeginCapture(h->b.s, hipStreamCaptureModeThreadLocal));
     const int rc = run_prog(h->b, which == 0 ? h->b.prog_step : h->b.prog_init);
-    const hipError_t e = hipStreamEndCapture(h->b.s, &h->graph[which]);
+    hipError_t e = hipStreamEndCapture(h->b.s, &h->graph[which]);
+    if (rc == F2D_OK && e == hipSuccess)
+      e = hipGraphInstantiate(&h->exec[which], h->graph[which], nullptr, nullptr, 0);
+    if (rc != F2D_OK || e != hipSuccess) {  // nothing is left half made
+      if (h->graph[which]) (void)hipGraphDestroy(h->graph[which]);
+      h->graph[which] = nullptr;
+      h->exec[which] = nullptr;
+    }
     if (rc) return rc;
     ECHK(e);
-    ECHK(hipGraphInstantiate(&h->exec[which], h->graph[which], nullptr, nullptr, 0));
   }
   ECHK(hipGraphLaunch(h->exec[which], s));
   return F2D_OK;
