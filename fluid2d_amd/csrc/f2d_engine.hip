@@ -3189,7 +3189,10 @@ constexpr int RB2_TILES = 256, RB2_TY_SMALL = 4;
 // the register coarse kernel: levels of at most COARSE_CELLS cells (halo
 // included) keep host copies of operator and mask, from which its operands
 // are packed
-constexpr int COARSE_TOP_CELLS = 2048;  // most cells of its top level
+// most cells of its top level: strips of 8 rows past 1024 only for FP32
+// operators (no FP64 hierarchy has that top level within the LDS budget, whose
+// rule picks it: the smallest, 48 x 24, needs 161488 of 159744 bytes)
+constexpr int COARSE_TOP_CELLS[2] = {1024, 2048};
 constexpr size_t COARSE_CELLS = (size_t)(64 + 2 * NH) * (64 + 2 * NH);
 
 // ---- task helpers ----------------------------------------------------------
@@ -4222,13 +4225,18 @@ static int run_prog_t(Batch& b, const std::vector<Launch>& prog, ProfSel* prof =
       case L_COARSE:
         if (L.creg > 0) {
           // creg - 1: the first slot of the launch's instances
-          if (L.creg == 1 && L.mode == 0)
-            F2D_LAUNCH((k_coarse_reg<T, true, 0>), dim3(g), B1, L.shmem, b.s, TK, b.dC, b.dPk, Q,
-                       b.dD, L.pred, L.inst0, 0);
-          else if (L.creg == 1)
-            F2D_LAUNCH((k_coarse_reg<T, true, 1>), dim3(g), B1, L.shmem, b.s, TK, b.dC, b.dPk, Q,
-                       b.dD, L.pred, L.inst0, 0);
-          else if (L.mode == 0)
+          if constexpr (sizeof(T) == 4) {
+            if (L.creg == 1) {
+              if (L.mode == 0)
+                F2D_LAUNCH((k_coarse_reg<T, true, 0>), dim3(g), B1, L.shmem, b.s, TK, b.dC, b.dPk,
+                           Q, b.dD, L.pred, L.inst0, 0);
+              else
+                F2D_LAUNCH((k_coarse_reg<T, true, 1>), dim3(g), B1, L.shmem, b.s, TK, b.dC, b.dPk,
+                           Q, b.dD, L.pred, L.inst0, 0);
+              break;
+            }
+          }
+          if (L.mode == 0)
             F2D_LAUNCH((k_coarse_reg<T, false, 0>), dim3(g), B1, L.shmem, b.s, TK, b.dC, b.dPk, Q,
                        b.dD, L.pred, L.inst0, L.creg - 1);
           else
@@ -4789,7 +4797,7 @@ static void coarse_desc(const Batch& b, HostInst& h, int k0, double* pk) {
     N[l] = d.L[l].n - 2 * NH;
   }
   coarse::Desc& c = h.cd;
-  h.creg = coarse::slots(k0, d.nlev, M, N, COARSE_TOP_CELLS, &c.top, &c.deep);
+  h.creg = coarse::slots(k0, d.nlev, M, N, COARSE_TOP_CELLS[b.prec], &c.top, &c.deep);
   if (!h.creg) return;
   const size_t tsz = b.prec == 0 ? sizeof(double) : sizeof(float);
   int v = 0;
@@ -4849,14 +4857,15 @@ static int apply_tuning(Batch& b, const f2d_batch_tuning* t) {
     if (b.H[i].creg)
       reglds = std::max(reglds, coarse::lds_values(b.H[i].cd) * sizeof(double));
   if (reglds > 65536) {
-    const void* fn[8] = {
-        (const void*)k_coarse_reg<double, false, 0>, (const void*)k_coarse_reg<double, true, 0>,
-        (const void*)k_coarse_reg<double, false, 1>, (const void*)k_coarse_reg<double, true, 1>,
-        (const void*)k_coarse_reg<float, false, 0>,  (const void*)k_coarse_reg<float, true, 0>,
-        (const void*)k_coarse_reg<float, false, 1>,  (const void*)k_coarse_reg<float, true, 1>};
-    for (int q = 0; q < 4; q++)
-      ECHK(hipFuncSetAttribute(fn[4 * b.prec + q], hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)reglds));
+    const std::vector<const void*> fn =
+        b.prec == 0 ? std::vector<const void*>{(const void*)k_coarse_reg<double, false, 0>,
+                                               (const void*)k_coarse_reg<double, false, 1>}
+                    : std::vector<const void*>{(const void*)k_coarse_reg<float, false, 0>,
+                                               (const void*)k_coarse_reg<float, true, 0>,
+                                               (const void*)k_coarse_reg<float, false, 1>,
+                                               (const void*)k_coarse_reg<float, true, 1>};
+    for (const void* f : fn)
+      ECHK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)reglds));
   }
   std::vector<InstD> di(b.ninst);
   for (int i = 0; i < b.ninst; i++) di[i] = b.H[i].d;
