@@ -904,20 +904,29 @@ static int red_scratch(double** partial) {
 
 // Results of the calling thread's reductions in pinned host memory, which
 // every device writes: one synchronization of the null stream instead of an
-// allocation, a copy and a free for each scalar (2048 x 1024, a pass of seven
+// allocation, a copy and a free for each scalar (2048 x 1024, a pass of six
 // reductions: 208 us with those, 140 so).  A thread keeps its eight values
 // until it ends, then they go to the next thread that asks.
 namespace {
 constexpr int kScalars = 8;
-std::mutex g_scalars_mu;
-std::vector<double*> g_scalars_free;
+// the values of threads that have ended; never destroyed, for a thread may end
+// after the process's static objects (a daemon thread at exit)
+struct ScalarPool {
+  std::mutex mu;
+  std::vector<double*> free;
+};
+ScalarPool& scalar_pool() {
+  static ScalarPool* p = new ScalarPool();
+  return *p;
+}
 struct ThreadScalars {
   double* p = nullptr;
   ~ThreadScalars() {
     if (!p) return;
-    std::lock_guard<std::mutex> lk(g_scalars_mu);
+    ScalarPool& pool = scalar_pool();
+    std::lock_guard<std::mutex> lk(pool.mu);
     try {
-      g_scalars_free.push_back(p);
+      pool.free.push_back(p);
     } catch (...) {
     }
   }
@@ -928,10 +937,11 @@ thread_local ThreadScalars t_scalars;
 int f2d_scalars_f64(double** out) {
   double*& p = t_scalars.p;
   if (!p) {
-    std::lock_guard<std::mutex> lk(g_scalars_mu);
-    if (!g_scalars_free.empty()) {
-      p = g_scalars_free.back();
-      g_scalars_free.pop_back();
+    ScalarPool& pool = scalar_pool();
+    std::lock_guard<std::mutex> lk(pool.mu);
+    if (!pool.free.empty()) {
+      p = pool.free.back();
+      pool.free.pop_back();
     }
   }
   if (!p) {
