@@ -54,12 +54,16 @@ class Request:
         return Param(**kw)
 
     def est_bytes(self, precision):
-        """Device memory of one instance (state, tendencies, multigrid)."""
+        """Device memory of one instance: state, tendencies, multigrid, and
+        with the default launch shapes its share of the task lists (160 bytes
+        a tile of every launch; grids up to 512^2 run in tiles of 4 rows) and
+        the packed operands of the coarse levels."""
         cells = (self.n + 6) ** 2
         nvar = 5 if self.modelname == "euler" else 6
         tz = 8 if precision == "fp64" else 4
         pw = nvar + 8 + (0 if precision == "fp64" else 3)  # FP64 pool words per cell
-        return int(1.15 * cells * (8 * pw + tz * (3 * nvar + 3 + 11) + 5))
+        arrays = cells * (8 * pw + tz * (3 * nvar + 3 + 11) + 5)
+        return int(max(1.15 * arrays, arrays + 1.1 * 2 ** 20 + min(64 * cells, 16 << 20)))
 
 
 def stream_requests(count, rate=50.0, seed=5, sizes_log2=(7, 11), steps=(50, 2000)):
