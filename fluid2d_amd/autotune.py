@@ -1,6 +1,6 @@
 """Launch-configuration autotuner for the batched engine.
 
-Two knobs shape the launches of a batch (``f2d_batch_tuning``):
+These knobs shape the launches of a batch (``f2d_batch_tuning``):
 
 * ``coarse_lds_budget``: how many of the coarse multigrid levels the
   one-workgroup coarse kernel takes over (its operands must fit in LDS);
@@ -8,9 +8,9 @@ Two knobs shape the launches of a batch (``f2d_batch_tuning``):
 * ``min_tiles``: the fine phases use 64 x 16, 64 x 8 or 64 x 4 tiles, the
   tallest that still gives this many workgroups, so that small levels
   spread over more compute units (0: the default, 1024; 1: always 16 rows).
-* ``coarse_wave_cells``: inside the coarse kernel, levels up to this size
-  run on a single wavefront (no workgroup barriers) instead of the whole
-  workgroup.
+* ``coarse_wave_cells``: inside the generic coarse kernel, levels up to this
+  size run on a single wavefront (no workgroup barriers) instead of the whole
+  workgroup.  Tried only where a batch launches that kernel.
 * ``persist``: runs of consecutive smoother and residual/restriction phases
   below the finest level run as one persistent launch with device-wide
   barriers (at most this many workgroups per compute unit), or one launch
@@ -118,10 +118,16 @@ def tune(specs, precision="fp64", steps=3, cands=None, use_cache=True, verbose=F
     b = Batch(pg, precision=precision)
     _init(b)
     table = []
+    same = set()  # candidates without coarse_wave_cells, where it changes nothing
 
     def trial(c):
+        key = tuple(sorted((k, v) for k, v in c.items() if k != "coarse_wave_cells"))
+        if key in same:
+            return
         try:
             b.retune(c)
+            if b.coarse_generic() == 0:
+                same.add(key)
             b.step(1)  # capture + warm
             t0 = time.perf_counter()
             b.step(steps)

@@ -31,6 +31,7 @@ _SIG = {
     "f2d_batch_retune": ([_p, _p], _i),
     "f2d_batch_tuning_info": ([_p, _p], _i),
     "f2d_batch_destroy": ([_p], _i),
+    "f2d_batch_coarse_generic": ([_p, C.POINTER(_i)], _i),
     "f2d_batch_info": ([_p, _i, C.POINTER(_i), C.POINTER(_i), C.POINTER(C.c_longlong)], _i),
     "f2d_batch_set_field": ([_p, _i, _i, _p], _i),
     "f2d_batch_get_state": ([_p, _i, _p], _i),
@@ -86,9 +87,10 @@ def _call(name, *args):
 class Tuning(C.Structure):
     """f2d_batch_tuning: coarse-kernel LDS budget (bytes, 0 = device
     maximum), the minimum workgroup count of a fine phase (0 = default 1024,
-    1 = always 16-row tiles), the largest coarse level (cells) run on one wavefront
-    (-1 = default 256) and the persistent multigrid launches (workgroups per
-    compute unit, 0 = one launch per phase)."""
+    1 = always 16-row tiles), the largest coarse level (cells) the generic
+    coarse kernel runs on one wavefront (-1 = default 256) and the persistent
+    multigrid launches (workgroups per compute unit, 0 = one launch per
+    phase)."""
     _fields_ = [("coarse_lds_budget", C.c_int), ("min_tiles", C.c_int),
                 ("coarse_wave_cells", C.c_int), ("persist", C.c_int)]
 
@@ -221,6 +223,13 @@ class Batch:
         nl, nf, nlaunch = C.c_int(), C.c_int(), C.c_longlong()
         _call("f2d_batch_info", self._h, i, C.byref(nl), C.byref(nf), C.byref(nlaunch))
         return {"nlev": nl.value, "nfine": nf.value, "launches_per_step": nlaunch.value}
+
+    def coarse_generic(self):
+        """Launches of a step that run the generic coarse kernel (0: all run
+        the register one, which ``coarse_wave_cells`` does not concern)."""
+        n = C.c_int()
+        _call("f2d_batch_coarse_generic", self._h, C.byref(n))
+        return n.value
 
     def set_field(self, i, name, a):
         k = self.varnames[i].index(name)

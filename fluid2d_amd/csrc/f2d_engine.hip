@@ -5319,6 +5319,12 @@ int f2d_batch_info(f2d_batch* b, int inst, int* nlev, int* nfine, long long* lau
   return F2D_OK;
 }
 
+int f2d_batch_coarse_generic(f2d_batch* b, int* launches) {
+  *launches = 0;
+  for (const Launch& L : b->prog_step) *launches += L.kind == L_COARSE && L.creg == 0;
+  return F2D_OK;
+}
+
 int f2d_batch_set_field(f2d_batch* b, int inst, int field, const double* host) {
   if (inst < 0 || inst >= b->ninst) return efail(F2D_E_ARG, "instance out of range");
   const InstD& d = b->H[inst].d;

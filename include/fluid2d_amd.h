@@ -290,10 +290,13 @@ const char *f2d_batch_last_error(void);
  * min_tiles: a fine-level phase uses the tallest tile (16, 8 or 4 rows of
  *   64 cells) that still gives at least this many workgroups (0 = the
  *   default, 1024; 1 = always 16 rows).
- * coarse_wave_cells: inside the coarse kernel, levels of at most this many
- *   cells (halo included) run on one wavefront without workgroup barriers;
- *   larger ones use the whole workgroup (0 = none on one wavefront;
- *   negative = the default, 256).
+ * coarse_wave_cells: inside the generic coarse kernel, levels of at most this
+ *   many cells (halo included) run on one wavefront without workgroup
+ *   barriers; larger ones use the whole workgroup (0 = none on one wavefront;
+ *   negative = the default, 256).  Without effect on launches of the register
+ *   coarse kernel, which take the batches whose coarse levels all fit its
+ *   slots: coarsest level of at most 64 cells and 16 columns, top level of at
+ *   most 64 columns (f2d_batch_coarse_generic).
  * persist: > 0 runs each run of consecutive smoother and
  *   residual/restriction phases below the finest level as one persistent
  *   launch of at most `persist` workgroups per compute unit, with a bounded
@@ -321,6 +324,8 @@ int f2d_batch_retune(f2d_batch *b, const f2d_batch_tuning *tuning);
 int f2d_batch_tuning_info(f2d_batch *b, f2d_batch_tuning *out);
 int f2d_batch_destroy(f2d_batch *b);
 int f2d_batch_info(f2d_batch *b, int inst, int *nlev, int *nfine, long long *launches_per_step);
+/* launches of a step that run the generic coarse kernel */
+int f2d_batch_coarse_generic(f2d_batch *b, int *launches);
 int f2d_batch_set_field(f2d_batch *b, int inst, int field, const double *host);
 int f2d_batch_get_state(f2d_batch *b, int inst, double *host);
 int f2d_batch_state_ptr(f2d_batch *b, int inst, double **dev);
